@@ -22,6 +22,7 @@
 #include "grid.hpp"
 #include "dft.hpp"
 #include "kernels.hpp"
+#include "p2p.hpp"
 #include "plan.hpp"
 #include "xfer.hpp"
 
@@ -1595,11 +1596,9 @@ __global__ __launch_bounds__(256) void k_l2p_mfma(
   }
 }
 
-// P2P near field (P2P.hpp:42-79): p_i += sum_j exp(i kappa r)/(4 pi r) q_j,
-// r = |x_i - y_j|, term 0 when r^2 < 1e-16.  A work item is up to 64 targets
-// of one leaf against a run of its source list; with nt targets, the wave's
-// lanes form floor(64/nt) groups that split the sources.  Sources are staged
-// in LDS 64 at a time.  Each item writes per-target partial sums (double).
+// P2P near field (P2P.hpp:42-79) on the matrix cores.  A work item is up to
+// 64 targets of one leaf against a run of its source list; it writes
+// per-target partial sums (double).
 struct P2PItem {
   int leaf;  // index into the leaf list
   int t0;    // first target of the chunk (leaf-relative)
@@ -1615,34 +1614,6 @@ struct P2PItem {
 template <typename R, bool Small>
 __device__ __forceinline__ void p2pKernel(double xt, double yt, double zt, double xs, double ys,
                                           double zs, double kappa, R& co, R& si);
-template <>
-__device__ __forceinline__ void p2pKernel<double, true>(double xt, double yt, double zt,
-                                                        double xs, double ys, double zs,
-                                                        double kappa, double& co, double& si) {
-  const double x = xt - xs, y = yt - ys, z = zt - zs;
-  const double R2v = x * x + y * y + z * z;
-  double K = rsqrt(R2v);
-  if (R2v < 1.e-16) K = 0.;
-  const double r = K * R2v * kappa;
-  K *= 0.079577471545947667884;  // 1/(4 pi)
-  sincosRedSmall(r, si, co);
-  co *= K;
-  si *= K;
-}
-template <>
-__device__ __forceinline__ void p2pKernel<double, false>(double xt, double yt, double zt,
-                                                         double xs, double ys, double zs,
-                                                         double kappa, double& co, double& si) {
-  const double x = xt - xs, y = yt - ys, z = zt - zs;
-  const double R2v = x * x + y * y + z * z;
-  double K = rsqrt(R2v);
-  if (R2v < 1.e-16) K = 0.;
-  const double r = K * R2v * kappa;
-  K *= 0.079577471545947667884;  // 1/(4 pi)
-  sincosRed(r, si, co);
-  co *= K;
-  si *= K;
-}
 template <>
 __device__ __forceinline__ void p2pKernel<float, true>(double xt, double yt, double zt,
                                                        double xs, double ys, double zs,
@@ -1677,123 +1648,10 @@ __device__ __forceinline__ void p2pKernel<float, true>(double xt, double yt, dou
   si *= K;
 }
 
-// NR right-hand sides: charges q + r * qStride; the partial sums of item k,
-// right-hand side r, lane t at partial[(k * NR + r) * 64 + t].
-template <typename R, int NR>
-__global__ __launch_bounds__(64) void k_p2p(const P2PItem* __restrict__ items,
-                                            const int* __restrict__ leafCell,
-                                            const int* __restrict__ tpbeg,
-                                            const int* __restrict__ tnprt,
-                                            const double* __restrict__ tx,
-                                            const double* __restrict__ ty,
-                                            const double* __restrict__ tz,
-                                            const double* __restrict__ sx,
-                                            const double* __restrict__ sy,
-                                            const double* __restrict__ sz,
-                                            const typename C2T<R>::T* __restrict__ q,
-                                            size_t qStride,
-                                            const int* __restrict__ rb, const int* __restrict__ re,
-                                            double kappa, int smallArg,
-                                            double2* __restrict__ partial, int nItems) {
-  typedef typename C2T<R>::T R2;
-  __shared__ double lx[64], ly[64], lz[64];
-  __shared__ R2 lq[NR][64];
-  __shared__ double2 red[NR][64];
-  const int item = itemIndex();
-  if (item >= nItems) return;
-  const P2PItem it = items[item];
-  const int c = leafCell[it.leaf];
-  const int tb = tpbeg[c] + it.t0;
-  const int nt = min(64, tnprt[c] - it.t0);
-  const int G = 64 / nt;
-  const int lane = threadIdx.x;
-  const int ti = lane % nt, g = lane / nt;
-  const bool active = g < G;
-  const double xt = tx[tb + ti], yt = ty[tb + ti], zt = tz[tb + ti];
-  double accr[NR], acci[NR];
-#pragma unroll
-  for (int k = 0; k < NR; k++) accr[k] = acci[k] = 0.;
-  int r = it.r, off = it.off;
-  for (int pos = 0; pos < it.cnt; pos += 64) {
-    const int tileN = min(64, it.cnt - pos);
-    __syncthreads();
-    if (lane < tileN) {
-      int rr = r, oo = off + lane;
-      int len = re[rr] - rb[rr];
-      while (oo >= len) {
-        oo -= len;
-        rr++;
-        len = re[rr] - rb[rr];
-      }
-      const int j = rb[rr] + oo;
-      lx[lane] = sx[j];
-      ly[lane] = sy[j];
-      lz[lane] = sz[j];
-#pragma unroll
-      for (int k = 0; k < NR; k++) lq[k][lane] = q[k * qStride + j];
-    }
-    {
-      int adv = tileN;
-      while (adv > 0) {
-        const int rem = re[r] - rb[r] - off;
-        if (adv < rem) {
-          off += adv;
-          adv = 0;
-        } else {
-          adv -= rem;
-          r++;
-          off = 0;
-        }
-      }
-    }
-    __syncthreads();
-    if (active) {
-      R pr[NR], pi[NR];
-#pragma unroll
-      for (int k = 0; k < NR; k++) pr[k] = pi[k] = 0;
-      auto term = [&](int j, auto small) {
-        R co, si;
-        p2pKernel<R, decltype(small)::value>(xt, yt, zt, lx[j], ly[j], lz[j], kappa, co, si);
-#pragma unroll
-        for (int k = 0; k < NR; k++) {
-          const R2 qs = lq[k][j];
-          pr[k] += co * qs.x - si * qs.y;
-          pi[k] += co * qs.y + si * qs.x;
-        }
-      };
-      if (smallArg) {
-#pragma unroll 2
-        for (int j = g; j < tileN; j += G) term(j, std::true_type());
-      } else {
-        for (int j = g; j < tileN; j += G) term(j, std::false_type());
-      }
-#pragma unroll
-      for (int k = 0; k < NR; k++) {
-        accr[k] += (double)pr[k];
-        acci[k] += (double)pi[k];
-      }
-    }
-  }
-#pragma unroll
-  for (int k = 0; k < NR; k++) red[k][lane] = make_double2(accr[k], acci[k]);
-  __syncthreads();
-  if (lane < nt) {
-#pragma unroll
-    for (int k = 0; k < NR; k++) {
-      double2 s = red[k][lane];
-      for (int gg = 1; gg < G; gg++) {
-        s.x += red[k][gg * nt + lane].x;
-        s.y += red[k][gg * nt + lane].y;
-      }
-      partial[((size_t)item * NR + k) * 64 + lane] = s;
-    }
-  }
-}
-
 // P2P for 16 right-hand sides per launch on the matrix cores (float, the
 // mixed-precision path).  An item's near-field sum is the product of the
 // kernel matrix G (targets x sources, complex, evaluated by the VALU one
-// element per lane, double phase reduction as in k_p2p) and the charge matrix
+// element per lane, phase reduced in double) and the charge matrix
 // Q (sources x 16 right-hand sides):
 //   P_re += G_re Q_re - G_im Q_im,   P_im += G_re Q_im + G_im Q_re,
 // four V_MFMA_F32_16X16X4_F32 per 4 sources.  Operand layouts of that
@@ -1804,7 +1662,7 @@ __global__ __launch_bounds__(64) void k_p2p(const P2PItem* __restrict__ items,
 // current K-step k, and ends holding right-hand side l % 16 of targets
 // 16 w + 4 (l / 16) + 0..3.  Sources are staged 64 at a time in LDS (the
 // charges as [source][right-hand side]); each 64-source tile's sums are added
-// to double accumulators (as k_p2p does) and the item's partial sums go to
+// to double accumulators and the item's partial sums go to
 // the layout k_p2p_reduce<float, 16> reads.
 constexpr int kP2PMfmaNR = 16;
 
@@ -1911,8 +1769,8 @@ __global__ __launch_bounds__(256) void k_p2p_mfma(
 
 // Sum the partial results of a leaf's items into p (items of a leaf are
 // contiguous, ordered by target chunk).
-// NR right-hand sides (partial layout of k_p2p<R, NR>); right-hand side r
-// adds into p + r * pStride.
+// NR right-hand sides (partial sums of item k, right-hand side r, target t at
+// partial[(k * NR + r) * 64 + t]); right-hand side r adds into p + r * pStride.
 template <typename R, int NR>
 __global__ __launch_bounds__(64) void k_p2p_reduce(const int* __restrict__ itemBeg,
                                                    const P2PItem* __restrict__ items,
@@ -2056,6 +1914,13 @@ struct Exec {
   int nTslots = 0, nSslots = 0;
   P2PItem* items = nullptr;
   int nitems = 0;
+  // items of the near field with a lane per source (p2p.hpp)
+  P2PLaneItem* laneItems = nullptr;
+  int nLaneItems = 0;
+  int* laneItemBeg = nullptr;
+  int p2pPhase = kPhaseLibrary;
+  PhaseConsts phaseConsts{};
+  void* phaseTab = nullptr;  // kPhaseN complex values, plan's real type
   int *leafCell = nullptr, *itemBeg = nullptr, *rb = nullptr, *re = nullptr;
   int nleaves = 0;
   double2* partial = nullptr;
@@ -2112,6 +1977,7 @@ struct Exec {
     ML = F = Lb = q = p = nullptr;
     gSrc = bRows = nullptr;
     partial = qio = pio = nullptr;
+    phaseTab = nullptr;
   }
   // wait until the last execution, on whatever stream, has finished
   int quiesce() {
@@ -2283,6 +2149,15 @@ __global__ void k_table_rows(const int* __restrict__ keys, int64_t nrows,
   }
 }
 
+// Partial sums of the near field: of one launch of the widest kernel that a
+// pass of X.nr right-hand sides uses.
+static size_t partialElems(const Exec& X) {
+  size_t n = (size_t)X.nLaneItems * std::min(X.nr, X.prec == DEFMM_MIXED ? 8 : 4) * kP2PTargets;
+  if (X.prec == DEFMM_MIXED && X.nr >= kP2PMfmaNR)
+    n = std::max(n, (size_t)X.nitems * 64 * kP2PMfmaNR);
+  return std::max<size_t>(n, 1);
+}
+
 template <typename R>
 static int uploadTyped(Exec& X) {
   typedef typename C2T<R>::T R2;
@@ -2364,6 +2239,17 @@ static int uploadTyped(Exec& X) {
     CKR(X.upv(d, c));
     X.consts = d;
   }
+  {
+    std::vector<R2> t(kPhaseN);
+    for (int k = 0; k < kPhaseN; k++) {
+      double c, sn;
+      phaseEntry(k, c, sn);
+      t[k] = c2h<R>(c, sn);
+    }
+    R2* d;
+    CKR(X.upv(d, t));
+    X.phaseTab = d;
+  }
   // right-hand side r of every store at base + r * stride
   const size_t nr = (size_t)X.nr;
   if (X.m2lMode == DEFMM_M2L_STORED) {
@@ -2401,7 +2287,7 @@ static int uploadTyped(Exec& X) {
   CKR(X.alloc(X.p, nr * (size_t)X.nt * sizeof(R2)));
   {
     void* d;
-    CKR(X.alloc(d, nr * (size_t)std::max(1, X.nitems) * 64 * sizeof(double2)));
+    CKR(X.alloc(d, partialElems(X) * sizeof(double2)));
     X.partial = (double2*)d;
     CKR(X.alloc(d, nr * (size_t)X.ns * sizeof(double2)));
     X.qio = (double2*)d;
@@ -2427,8 +2313,8 @@ static int chooseM2LMode(Exec& X) {
     freeB = std::min(freeB, (size_t)std::max<int64_t>(0, X.memLimit - X.bytes));
   const size_t r2 = X.prec == DEFMM_FP64 ? 16 : 8;
   const size_t storedB =
-      (size_t)X.nr * (((size_t)X.nm2f * X.PP + X.nMLslots * X.LL) * r2 + ((size_t)X.ns + X.nt) * (r2 + 16) +
-                      (size_t)X.nitems * 64 * 16) +
+      (size_t)X.nr * (((size_t)X.nm2f * X.PP + X.nMLslots * X.LL) * r2 + ((size_t)X.ns + X.nt) * (r2 + 16)) +
+      partialElems(X) * sizeof(double2) +
       (size_t)X.hGSrcF.size() * sizeof(int);
   X.m2lMode = (double)storedB < 0.9 * (double)freeB ? DEFMM_M2L_STORED : DEFMM_M2L_BATCHED;
   return OK;
@@ -2470,6 +2356,66 @@ static int reupload(Exec& X, int oldNr, int oldPrec, int oldMode, bool oldAuto, 
   return rc;
 }
 
+// Items of the near field with a lane per source: a leaf's targets in equal
+// chunks of at most kP2PTargets, its source list in equal runs (multiples of
+// 64) of at most `budget` sources.  8,192 sources a run amortise the final
+// sum over the wave; where that leaves fewer than 16,384 items (16 waves per
+// SIMD's share of the chip are needed to hide latency and even out the end)
+// the budget is halved, down to 512.
+static int buildLaneItems(Exec& X, const Plan& pl) {
+  const Tree& T = pl.T;
+  const size_t nl = pl.p2pLeaf.size();
+  std::vector<P2PLaneItem> items;
+  std::vector<int> beg;
+  std::vector<int64_t> total(nl, 0);
+  for (size_t lf = 0; lf < nl; lf++)
+    for (int r = pl.p2pBeg[lf]; r < pl.p2pBeg[lf + 1]; r++)
+      total[lf] += pl.p2pSrcE[r] - pl.p2pSrcB[r];
+  auto chunksOf = [&](size_t lf) { return (T.nprt[pl.p2pLeaf[lf]] + kP2PTargets - 1) / kP2PTargets; };
+  int64_t budget = 8192;
+  for (;; budget /= 2) {
+    int64_t n = 0;
+    for (size_t lf = 0; lf < nl; lf++) n += chunksOf(lf) * ((total[lf] + budget - 1) / budget);
+    if (n > INT32_MAX / 2) {
+      g_err = "near-field work items exceed the launch index range";
+      return ERR_ARG;
+    }
+    if (n >= 16384 || budget <= 512) {
+      items.reserve((size_t)n);
+      break;
+    }
+  }
+  for (size_t lf = 0; lf < nl; lf++) {
+    beg.push_back((int)items.size());
+    const int n = T.nprt[pl.p2pLeaf[lf]], chunks = chunksOf(lf);
+    const int64_t runs = (total[lf] + budget - 1) / budget;
+    if (runs == 0 || chunks == 0) continue;
+    const int chunk = (n + chunks - 1) / chunks;
+    const int64_t len = ((total[lf] + runs - 1) / runs + 63) / 64 * 64;
+    int r = pl.p2pBeg[lf], off = 0;
+    for (int64_t pos = 0; pos < total[lf]; pos += len) {
+      const int cnt = (int)std::min(len, total[lf] - pos);
+      while (off >= pl.p2pSrcE[r] - pl.p2pSrcB[r]) {
+        off -= pl.p2pSrcE[r] - pl.p2pSrcB[r];
+        r++;
+      }
+      for (int t0 = 0; t0 < n; t0 += chunk)
+        items.push_back({(int)lf, t0, std::min(chunk, n - t0), r, off, cnt});
+      off += cnt;
+    }
+    // the reduction counts ceil(n / kP2PTargets) items per run
+    if (((int)items.size() - beg.back()) % chunks != 0) {
+      g_err = "internal: near-field items do not match the leaf's chunks";
+      return ERR_STATE;
+    }
+  }
+  beg.push_back((int)items.size());
+  X.nLaneItems = (int)items.size();
+  CKR(X.upv(X.laneItems, items));
+  CKR(X.upv(X.laneItemBeg, beg));
+  return OK;
+}
+
 static int upload(Exec& X, Plan& pl) {
   X.L = pl.L; X.P = pl.P; X.LL = pl.LL; X.PP = pl.PP; X.kappa = pl.kappa;
   {
@@ -2488,6 +2434,8 @@ static int upload(Exec& X, Plan& pl) {
     for (int d = 0; d < 3; d++) diag2 += (hi[d] - lo[d]) * (hi[d] - lo[d]);
     X.smallArg = std::fabs(pl.kappa) * std::sqrt(diag2) * (1. + 1e-12) <= 1048576.0 ? 1 : 0;
   }
+  X.p2pPhase = phaseOf(X.kappa, X.smallArg != 0);
+  X.phaseConsts = phaseConstsOf(X.kappa);
   X.st = pl.st;
   X.ns = (int64_t)pl.S.x.size();
   X.nt = (int64_t)pl.T.x.size();
@@ -2704,6 +2652,9 @@ static int upload(Exec& X, Plan& pl) {
     X.st.p2p_items = X.nitems;
     CKR(X.upv(X.items, items));
     CKR(X.upv(X.itemBeg, itemBeg));
+  }
+  CKR(buildLaneItems(X, pl));
+  {
     CKR(X.upv(X.leafCell, pl.p2pLeaf));
     CKR(X.upv(X.rb, pl.p2pSrcB));
     CKR(X.upv(X.re, pl.p2pSrcE));
@@ -2763,16 +2714,24 @@ static int m2lChunk(Exec& X, hipStream_t s, int g0, int ng, int r0, int n, const
   return 1;
 }
 
+// NR right-hand sides with a lane per source
 template <typename R, int NR>
-static void launchP2P(Exec& X, hipStream_t s, int r0) {
+static void launchP2PLane(Exec& X, hipStream_t s, int r0) {
   typedef typename C2T<R>::T R2;
   const R2* q = (const R2*)X.q + (size_t)r0 * X.ns;
   R2* p = (R2*)X.p + (size_t)r0 * X.nt;
-  hipLaunchKernelGGL((k_p2p<R, NR>), itemGrid(X.nitems), dim3(64), 0, s, X.items, X.leafCell,
-                     X.T.pbeg, X.T.nprt, X.tx, X.ty, X.tz, X.sx, X.sy, X.sz, q, (size_t)X.ns, X.rb,
-                     X.re, X.kappa, X.smallArg, X.partial, X.nitems);
-  hipLaunchKernelGGL((k_p2p_reduce<R, NR>), itemGrid(X.nleaves), dim3(64), 0, s, X.itemBeg,
-                     X.items, X.leafCell, X.T.pbeg, X.T.nprt, (const double2*)X.partial, p,
+  auto go = [&](auto phase) {
+    hipLaunchKernelGGL((k_p2p_lane<R, NR, decltype(phase)::value>),
+                       itemGrid(((int64_t)X.nLaneItems + 3) / 4), dim3(256), 0, s, X.laneItems,
+                       X.leafCell, X.T.pbeg, X.tx, X.ty, X.tz, X.sx, X.sy, X.sz, q, (size_t)X.ns,
+                       X.rb, X.re, (const R2*)X.phaseTab, X.phaseConsts, X.partial,
+                       X.nLaneItems);
+  };
+  if (X.p2pPhase == kPhaseNone) go(std::integral_constant<int, kPhaseNone>());
+  else if (X.p2pPhase == kPhaseTable) go(std::integral_constant<int, kPhaseTable>());
+  else go(std::integral_constant<int, kPhaseLibrary>());
+  hipLaunchKernelGGL((k_p2p_lane_reduce<R, NR>), itemGrid(X.nleaves), dim3(64), 0, s,
+                     X.laneItemBeg, X.leafCell, X.T.pbeg, X.T.nprt, (const double2*)X.partial, p,
                      (size_t)X.nt, X.nleaves);
 }
 
@@ -2950,18 +2909,20 @@ static int runTyped(Exec& X, const double2* qin, double2* pout, int parts, int n
   mark(7);
   if (near && X.nitems) {
     // near field: per-item partial sums, then folded into p per target leaf,
-    // up to 8 right-hand sides per kernel value on the VALU, 16 on the
-    // matrix cores in float.  (Run on a second stream beside M2L it measured
+    // up to 8 right-hand sides per kernel value on the VALU (double: 4, whose
+    // sums fit the registers; two launches of 4 take 1.02 ms at 20,000 points
+    // where one of 8 took 1.41), 16 on the matrix cores in float.  (Run on a second stream beside M2L it measured
     // no faster: both contend for the same CUs.)
     for (int r0 = 0; r0 < nrhs;) {
       const int n = nrhs - r0;
       if (sizeof(R) == 4 && n >= kP2PMfmaNR && X.p2pMfma) {
         launchP2PMfma(X, s, r0);
         r0 += kP2PMfmaNR;
-      } else if (n >= 8) { launchP2P<R, 8>(X, s, r0); r0 += 8; }
-      else if (n >= 4) { launchP2P<R, 4>(X, s, r0); r0 += 4; }
-      else if (n >= 2) { launchP2P<R, 2>(X, s, r0); r0 += 2; }
-      else { launchP2P<R, 1>(X, s, r0); r0 += 1; }
+      } else if (sizeof(R) == 4 && n >= 8) { launchP2PLane<R, 8>(X, s, r0); r0 += 8; }
+      else if (n >= 4) { launchP2PLane<R, 4>(X, s, r0); r0 += 4; }
+      else if (n == 3) { launchP2PLane<R, 3>(X, s, r0); r0 += 3; }
+      else if (n >= 2) { launchP2PLane<R, 2>(X, s, r0); r0 += 2; }
+      else { launchP2PLane<R, 1>(X, s, r0); r0 += 1; }
     }
   }
   mark(8);
