@@ -136,6 +136,93 @@ DFM_UNROLL
     for (int k2 = 0; k2 < 5; k2++) x[(10 * k1 + 6 * k2) % 15] = a[k1][k2];
 }
 
+// Lines of the 3D transforms for any order L, P = 2L - 1; c[m], s[m] are cos
+// and sin of 2 pi m / P for m < L.  P = 15 takes the prime-factor transform;
+// the others use that cos is even and sin odd in m: the terms v and P - v of
+// an inverse line, and the outputs k and P - k of a forward one, share their
+// products, 4 (L - 1)^2 multiply-adds a line against 4 L P of the direct sum.
+constexpr int dftIndex(int m, int P) { return m % P <= P / 2 ? m % P : P - m % P; }
+constexpr bool dftFlip(int m, int P) { return m % P > P / 2; }
+
+// y_k = sum_{j < L} x_j exp(-2 pi i j k / P), k < P
+template <int L, typename R, typename T2>
+DFM_HD_INLINE void dftForward(const T2 (&x)[L], T2 (&y)[2 * L - 1], const R (&c)[L],
+                              const R (&s)[L]) {
+  constexpr int P = 2 * L - 1;
+  if constexpr (P == 15) {
+DFM_UNROLL
+    for (int j = 0; j < L; j++) y[j] = x[j];
+    dft15<-1, L>(y);
+  } else {
+    T2 t = x[0];
+DFM_UNROLL
+    for (int j = 1; j < L; j++) {
+      t.x += x[j].x;
+      t.y += x[j].y;
+    }
+    y[0] = t;
+DFM_UNROLL
+    for (int k = 1; k < L; k++) {
+      T2 a = x[0], b;
+      b.x = b.y = (R)0;
+DFM_UNROLL
+      for (int j = 1; j < L; j++) {
+        const R cm = c[dftIndex(j * k, P)];
+        const R sm = dftFlip(j * k, P) ? -s[dftIndex(j * k, P)] : s[dftIndex(j * k, P)];
+        a.x += cm * x[j].x;
+        a.y += cm * x[j].y;
+        b.x += sm * x[j].x;
+        b.y += sm * x[j].y;
+      }
+      // a -+ i b
+      y[k].x = a.x + b.y;
+      y[k].y = a.y - b.x;
+      y[P - k].x = a.x - b.y;
+      y[P - k].y = a.y + b.x;
+    }
+  }
+}
+
+// y_k = sum_{v < P} x_v exp(+2 pi i v k / P), k < L
+template <int L, typename R, typename T2>
+DFM_HD_INLINE void dftInverse(const T2 (&x)[2 * L - 1], T2 (&y)[L], const R (&c)[L],
+                              const R (&s)[L]) {
+  constexpr int P = 2 * L - 1;
+  if constexpr (P == 15) {
+    T2 z[P];
+DFM_UNROLL
+    for (int v = 0; v < P; v++) z[v] = x[v];
+    dft15<1, P>(z);
+DFM_UNROLL
+    for (int k = 0; k < L; k++) y[k] = z[k];
+  } else {
+    T2 a[L], b[L];  // x_v +- x_{P-v}
+    T2 t = x[0];
+DFM_UNROLL
+    for (int v = 1; v < L; v++) {
+      a[v].x = x[v].x + x[P - v].x;
+      a[v].y = x[v].y + x[P - v].y;
+      b[v].x = x[v].x - x[P - v].x;
+      b[v].y = x[v].y - x[P - v].y;
+      t.x += a[v].x;
+      t.y += a[v].y;
+    }
+    y[0] = t;
+DFM_UNROLL
+    for (int k = 1; k < L; k++) {
+      T2 u = x[0];
+DFM_UNROLL
+      for (int v = 1; v < L; v++) {
+        const R cm = c[dftIndex(v * k, P)];
+        const R sm = dftFlip(v * k, P) ? -s[dftIndex(v * k, P)] : s[dftIndex(v * k, P)];
+        u.x += cm * a[v].x - sm * b[v].y;
+        u.y += cm * a[v].y + sm * b[v].x;
+      }
+      y[k] = u;
+    }
+  }
+}
+
 }  // namespace dfm
 
 #endif

@@ -589,6 +589,17 @@ __global__ __launch_bounds__(transLinesTB<L>()) void k_trans_lines(
 }
 
 
+// cos and sin of 2 pi m / P, m < L, of the plan's constants
+template <typename R, int L>
+__device__ __forceinline__ void loadTwiddles(const R* __restrict__ twc, const R* __restrict__ tws,
+                                             R (&cw)[L], R (&sw)[L]) {
+#pragma unroll
+  for (int m = 0; m < L; m++) {
+    cw[m] = twc[m];
+    sw[m] = tws[m];
+  }
+}
+
 // M2F (M2F.hpp:35-46, circulant.hpp:95-106): F = DFT_P^3 of M embedded in
 // the (2L-1)^3 grid at I2i(I, P), unnormalised, exp(-2 pi i jk/P).  The
 // embedding is zero outside the L^3 corner, so the three axis passes sum over
@@ -602,11 +613,12 @@ constexpr int m2fRows() {
   constexpr int r = 49152 / bytes;
   return r < 1 ? 1 : r > 4 ? 4 : r;
 }
-// Each pass gives one lane a whole line along its axis: the lane reads the
-// line's L inputs once and forms all P outputs, with twiddles whose indices
-// are compile-time constants (held in registers, not read from LDS); the last
-// pass stores F straight from registers.  For P = 15 (order 8) a line is the
-// prime-factor 15-point DFT of dft.hpp (168 instead of 480 operations).
+// Each pass gives one lane a whole line along its axis (dft.hpp): the lane
+// reads the line's L inputs once and forms all P outputs, with twiddles whose
+// indices are compile-time constants (held in registers, not read from LDS);
+// the last pass stores F straight from registers.  Lines that share the
+// products of k and P - k: float at L = 7 (a million points, 756,000 rows)
+// 4.7 -> 2.9 ms; where it is bound by writing F (double) it stays at 4.8 TB/s.
 template <typename R, int L>
 // Blocks for all nrhs right-hand sides of a launch: block b transforms rows
 // of right-hand side b / (blocks per right-hand side) (M + r * mStride into
@@ -629,90 +641,42 @@ __global__ __launch_bounds__(256) void k_m2f(const int* __restrict__ m2fSlot,
   F += rhs * fStride;
   const int row0 = (bi - rhs * perRhs) * NR;
   const int nr = min(NR, nRows - row0);
-  R cw[P], sw[P];
-#pragma unroll
-  for (int m = 0; m < P; m++) {
-    cw[m] = twc[m];
-    sw[m] = tws[m];
-  }
-  // t += v * exp(-2 pi i m / P)
-  auto mac = [&](R2& t, const R2 v, const int m) {
-    t.x += v.x * cw[m] + v.y * sw[m];
-    t.y += v.y * cw[m] - v.x * sw[m];
-  };
+  R cw[L], sw[L];
+  loadTwiddles<R, L>(twc, tws, cw, sw);
   // axis 2: line (k, i0, i1) of M -> T1[k][(i0 * L + i1) * P + k2]
   for (int x = tid; x < nr * L * L; x += 256) {
     const int k = x / (L * L), r = x - k * (L * L);
     const R2* Mr = M + (size_t)m2fSlot[row0 + k] * LL + r * L;
-    R2 v[L];
+    R2 v[L], y[P];
 #pragma unroll
     for (int j = 0; j < L; j++) v[j] = Mr[j];
-    if constexpr (P == 15) {
-      R2 y[P];
+    dftForward<L, R>(v, y, cw, sw);
 #pragma unroll
-      for (int j = 0; j < L; j++) y[j] = v[j];
-      dft15<-1, L>(y);
-#pragma unroll
-      for (int k2 = 0; k2 < P; k2++) T1[k][r * P + k2] = y[k2];
-    } else {
-#pragma unroll
-      for (int k2 = 0; k2 < P; k2++) {
-        R2 t = c2<R>(0, 0);
-#pragma unroll
-        for (int j = 0; j < L; j++) mac(t, v[j], (j * k2) % P);
-        T1[k][r * P + k2] = t;
-      }
-    }
+    for (int k2 = 0; k2 < P; k2++) T1[k][r * P + k2] = y[k2];
   }
   __syncthreads();
   // axis 1: line (k, i0, k2) -> T2[k][(i0 * P + k1) * P + k2]
   for (int x = tid; x < nr * L * P; x += 256) {
     const int k = x / (L * P), r = x - k * (L * P);
     const int i0 = r / P, k2 = r - i0 * P;
-    R2 v[L];
+    R2 v[L], y[P];
 #pragma unroll
     for (int j = 0; j < L; j++) v[j] = T1[k][(i0 * L + j) * P + k2];
-    if constexpr (P == 15) {
-      R2 y[P];
+    dftForward<L, R>(v, y, cw, sw);
 #pragma unroll
-      for (int j = 0; j < L; j++) y[j] = v[j];
-      dft15<-1, L>(y);
-#pragma unroll
-      for (int k1 = 0; k1 < P; k1++) T2[k][(i0 * P + k1) * P + k2] = y[k1];
-    } else {
-#pragma unroll
-      for (int k1 = 0; k1 < P; k1++) {
-        R2 t = c2<R>(0, 0);
-#pragma unroll
-        for (int j = 0; j < L; j++) mac(t, v[j], (j * k1) % P);
-        T2[k][(i0 * P + k1) * P + k2] = t;
-      }
-    }
+    for (int k1 = 0; k1 < P; k1++) T2[k][(i0 * P + k1) * P + k2] = y[k1];
   }
   __syncthreads();
   // axis 0: line (k, k1, k2) -> F[row0 + k][k0 * P^2 + k1 * P + k2]
   for (int x = tid; x < nr * P * P; x += 256) {
     const int k = x / (P * P), r = x - k * (P * P);
-    R2 v[L];
+    R2 v[L], y[P];
 #pragma unroll
     for (int j = 0; j < L; j++) v[j] = T2[k][j * P * P + r];
     R2* Fr = F + (size_t)(row0 + k) * PP + r;
-    if constexpr (P == 15) {
-      R2 y[P];
+    dftForward<L, R>(v, y, cw, sw);
 #pragma unroll
-      for (int j = 0; j < L; j++) y[j] = v[j];
-      dft15<-1, L>(y);
-#pragma unroll
-      for (int k0 = 0; k0 < P; k0++) Fr[k0 * P * P] = y[k0];
-    } else {
-#pragma unroll
-      for (int k0 = 0; k0 < P; k0++) {
-        R2 t = c2<R>(0, 0);
-#pragma unroll
-        for (int j = 0; j < L; j++) mac(t, v[j], (j * k0) % P);
-        Fr[k0 * P * P] = t;
-      }
-    }
+    for (int k0 = 0; k0 < P; k0++) Fr[k0 * P * P] = y[k0];
   }
 }
 
@@ -795,6 +759,63 @@ constexpr int m2lWavesPerEU() {
   return (L == 7 && sizeof(R) == 4) ? 6 : 1;
 }
 
+// F2L (F2L.hpp:35-46, circulant.hpp:108-118) of NB Fourier-domain expansions
+// staged in LDS (buf: NB x P^3, then work space; t1: NB x L P^2):
+//   dst_u[I] = inv * IDFT(J_u)[I2i(I, P)], only the L^3 corner.
+// A lane per line in each of the three sweeps, the lines of all NB together.
+// (Against a lane per output with twiddles read from LDS: M2L at order 6 and
+// 16 right-hand sides on 100,000 points 17.0 -> 13.2 ms, order 5 FP64 on
+// 200,000 points, where the rows' loads bound it, 31.4 -> 30.6 ms.)
+// Call with buf complete (after a barrier); buf and t1 are free again after
+// the caller's next barrier.
+template <typename R, int L, int TB, int NB>
+__device__ __forceinline__ void f2lLines(typename C2T<R>::T* buf, typename C2T<R>::T* t1,
+                                         typename C2T<R>::T* const (&dst)[NB], R inv,
+                                         const R (&cw)[L], const R (&sw)[L], int tid) {
+  typedef typename C2T<R>::T R2;
+  constexpr int P = 2 * L - 1, P2 = P * P, PP = P * P * P;
+  // axis 0: t1[u][(k0 * P + w1) * P + w2], k0 < L
+  for (int x = tid; x < NB * P2; x += TB) {
+    const int u = x / P2, r = x - u * P2;
+    R2 v[P], y[L];
+#pragma unroll
+    for (int w = 0; w < P; w++) v[w] = buf[u * PP + w * P2 + r];
+    dftInverse<L, R>(v, y, cw, sw);
+#pragma unroll
+    for (int k = 0; k < L; k++) t1[u * (L * P2) + k * P2 + r] = y[k];
+  }
+  __syncthreads();
+  // axis 1: buf[u][(k0 * L + k1) * P + w2], k1 < L
+  for (int x = tid; x < NB * L * P; x += TB) {
+    const int u = x / (L * P), z = x - u * (L * P);
+    const int k0 = z / P, w2 = z - k0 * P;
+    R2 v[P], y[L];
+#pragma unroll
+    for (int w = 0; w < P; w++) v[w] = t1[u * (L * P2) + (k0 * P + w) * P + w2];
+    dftInverse<L, R>(v, y, cw, sw);
+#pragma unroll
+    for (int k = 0; k < L; k++) buf[u * PP + (k0 * L + k) * P + w2] = y[k];
+  }
+  __syncthreads();
+  // axis 2 and scaling: dst[u][(k0 * L + k1) * L + k2]
+  for (int x = tid; x < NB * L * L; x += TB) {
+    const int u = x / (L * L), z = x - u * (L * L);
+    R2 v[P], y[L];
+#pragma unroll
+    for (int w = 0; w < P; w++) v[w] = buf[u * PP + z * P + w];
+    dftInverse<L, R>(v, y, cw, sw);
+    R2* d = dst[0];
+#pragma unroll
+    for (int k = 1; k < NB; k++) d = u == k ? dst[k] : d;
+    if (d)
+#pragma unroll
+      for (int k = 0; k < L; k++) d[z * L + k] = c2<R>(y[k].x * inv, y[k].y * inv);
+  }
+}
+// Expansions per f2lLines call: two fill more of the block's lanes (2 P^2
+// lines) without more LDS than the occupancy that the registers allow.
+constexpr int f2lBatch(int units) { return units < 2 ? units : 2; }
+
 template <int PP>
 __device__ __forceinline__ size_t tableRow(int code) {
   return (size_t)(code >> 3) * PP;
@@ -820,8 +841,8 @@ __attribute__((amdgpu_waves_per_eu(m2lWavesPerEU<R, L, NR>(), 8))) void k_m2l(
   typedef typename C2T<R>::T R2;
   constexpr int P = 2 * L - 1, LL = L * L * L, PP = P * P * P;
   constexpr int NW = M2LShapeN<L, NR>::NW, TB = M2LShapeN<L, NR>::TB, G = M2LShapeN<L, NR>::G;
-  __shared__ R2 J[PP], T1[L * P * P], T2[L * L * P];
-  __shared__ R wc[P], ws[P];
+  constexpr int NU = G * NR, NB = f2lBatch(NU);
+  __shared__ R2 J[NB * PP], T1[NB * L * P * P];
   const int tid = threadIdx.x;
   // Workgroups are dealt to the 8 XCDs round-robin; give each XCD a
   // contiguous part of the (direction-major) group order so that its L2 sees
@@ -831,10 +852,6 @@ __attribute__((amdgpu_waves_per_eu(m2lWavesPerEU<R, L, NR>(), 8))) void k_m2l(
   if (b >= nItems) return;
   const int n8 = nItems & ~7;
   const int grp = b < n8 ? (b & 7) * (n8 >> 3) + (b >> 3) : b;
-  if (tid < P) {
-    wc[tid] = twc[tid];
-    ws[tid] = tws[tid];
-  }
   // frequencies of this thread, clamped to PP - 1: every load is in bounds
   // and unconditional, and the accumulators of w >= PP are never stored
   unsigned wl[NW];
@@ -916,63 +933,30 @@ __attribute__((amdgpu_waves_per_eu(m2lWavesPerEU<R, L, NR>(), 8))) void k_m2l(
         for (int r = 0; r < NR; r++) cmacFma(acc[g][m][r], u[g][m], f[m][r]);
     }
   }
+  // F2L of the group's G x NR expansions, NB at a time
   const R inv = (R)(1.0 / (double)PP);
+  R cw[L], sw[L];
+  loadTwiddles<R, L>(twc, tws, cw, sw);
 #pragma unroll
-  for (int g = 0; g < G; g++) {
-    const int t = groupTarget[(size_t)grp * G + g];
-    if (t < 0) continue;
+  for (int u0 = 0; u0 < NU; u0 += NB) {
+    R2* dst[NB];
+    if (u0 > 0) __syncthreads();
 #pragma unroll
-    for (int rr = 0; rr < NR; rr++) {
-    R2* Lr = Lout + rr * lStride + (size_t)t * LL;
-    __syncthreads();
+    for (int j = 0; j < NB; j++) {
+      const int u = u0 + j;
+      dst[j] = nullptr;
+      if (u >= NU) continue;
+      const int g = u / NR, rr = u % NR;
+      const int t = groupTarget[(size_t)grp * G + g];
+      if (t >= 0) dst[j] = Lout + rr * lStride + (size_t)t * LL;
 #pragma unroll
-    for (int m = 0; m < NW; m++) {
-      const int w = tid + TB * m;
-      if (w < PP) J[w] = acc[g][m][rr];
-    }
-    __syncthreads();
-    // axis 0: T1[(k0*P + w1)*P + w2], k0 < L
-    for (int x = tid; x < L * P * P; x += TB) {
-      const int r = x % (P * P), k0 = x / (P * P);
-      R2 s = c2<R>(0, 0);
-#pragma unroll
-      for (int v0 = 0; v0 < P; v0++) {
-        const int m = (v0 * k0) % P;
-        const R2 v = J[v0 * P * P + r];
-        s.x += v.x * wc[m] - v.y * ws[m];
-        s.y += v.y * wc[m] + v.x * ws[m];
+      for (int m = 0; m < NW; m++) {
+        const int w = tid + TB * m;
+        if (w < PP) J[j * PP + w] = acc[g][m][rr];
       }
-      T1[x] = s;
     }
     __syncthreads();
-    // axis 1: T2[(k0*L + k1)*P + w2], k1 < L
-    for (int x = tid; x < L * L * P; x += TB) {
-      const int v2 = x % P, k1 = (x / P) % L, k0 = x / (L * P);
-      R2 s = c2<R>(0, 0);
-#pragma unroll
-      for (int v1 = 0; v1 < P; v1++) {
-        const int m = (v1 * k1) % P;
-        const R2 v = T1[(k0 * P + v1) * P + v2];
-        s.x += v.x * wc[m] - v.y * ws[m];
-        s.y += v.y * wc[m] + v.x * ws[m];
-      }
-      T2[x] = s;
-    }
-    __syncthreads();
-    // axis 2 and scaling: L[(k0*L + k1)*L + k2]
-    for (int x = tid; x < LL; x += TB) {
-      const int k2 = x % L, r = x / L;
-      R2 s = c2<R>(0, 0);
-#pragma unroll
-      for (int v2 = 0; v2 < P; v2++) {
-        const int m = (v2 * k2) % P;
-        const R2 v = T2[r * P + v2];
-        s.x += v.x * wc[m] - v.y * ws[m];
-        s.y += v.y * wc[m] + v.x * ws[m];
-      }
-      Lr[x] = c2<R>(s.x * inv, s.y * inv);
-    }
-    }
+    f2lLines<R, L, TB, NB>(J, T1, dst, inv, cw, sw, tid);
   }
 }
 
@@ -997,20 +981,16 @@ __global__ __launch_bounds__(M2LShape<L>::TB) void k_m2l_col(
   constexpr int P = 2 * L - 1, P2 = P * P, LL = L * L * L, PP = P * P * P;
   constexpr int TB = M2LShape<L>::TB;
   static_assert(M2LShape<L>::G == 1, "one target per group");
-  // order 8 runs each F2L step for all NR right-hand sides at once
+  // right-hand sides per F2L sweep: both at order 8, where their LDS still
+  // lets two blocks share a CU
   constexpr int NT = P == 15 ? NR : 1;
   __shared__ R2 T1[NT][L * P2], T2[NT][L * L * P];
-  __shared__ R wc[P], ws[P];
   const int tid = threadIdx.x;
   const int b = itemIndex();
   if (b >= nItems) return;
   // XCD-contiguous group order, as in k_m2l
   const int n8 = nItems & ~7;
   const int grp = b < n8 ? (b & 7) * (n8 >> 3) + (b >> 3) : b;
-  if (tid < P) {
-    wc[tid] = twc[tid];
-    ws[tid] = tws[tid];
-  }
   // threads beyond the cube's columns load a valid column and store nothing
   const int col = min(tid, P2 - 1);
   R2 acc[P][NR];
@@ -1041,91 +1021,44 @@ __global__ __launch_bounds__(M2LShape<L>::TB) void k_m2l_col(
   const int t = groupTarget[grp];
   if (t < 0) return;  // (uniform over the block)
   const R inv = (R)(1.0 / (double)PP);
-  if constexpr (P == 15) {
-    // prime-factor 15-point lines; each step for all right-hand sides, one
-    // barrier per step: axis 0 in registers, then a lane per line of axis 1
-    // (NR * L * P lines) and of axis 2 (NR * L^2 lines)
+  R cw[L], sw[L];
+  loadTwiddles<R, L>(twc, tws, cw, sw);
+  // NT right-hand sides at a time: axis 0 in registers, then a lane per line
+  // of axis 1 (NT * L * P lines) and of axis 2 (NT * L^2 lines)
+#pragma unroll
+  for (int r0 = 0; r0 < NR; r0 += NT) {
+    if (r0 > 0) __syncthreads();  // T1 and T2 of the previous ones consumed
     if (tid < P2)
 #pragma unroll
-      for (int rr = 0; rr < NR; rr++) {
-        R2 y[P];
+      for (int j = 0; j < NT; j++) {
+        R2 x[P], y[L];
 #pragma unroll
-        for (int m = 0; m < P; m++) y[m] = acc[m][rr];
-        dft15<1, P>(y);
+        for (int m = 0; m < P; m++) x[m] = acc[m][r0 + j];
+        dftInverse<L, R>(x, y, cw, sw);
 #pragma unroll
-        for (int k0 = 0; k0 < L; k0++) T1[rr][k0 * P2 + tid] = y[k0];
+        for (int k0 = 0; k0 < L; k0++) T1[j][k0 * P2 + tid] = y[k0];
       }
     __syncthreads();
-    for (int x = tid; x < NR * L * P; x += TB) {
-      const int rr = x / (L * P), z = x - rr * (L * P);
+    for (int x = tid; x < NT * L * P; x += TB) {
+      const int j = x / (L * P), z = x - j * (L * P);
       const int k0 = z / P, v2 = z - k0 * P;
-      R2 y[P];
+      R2 v[P], y[L];
 #pragma unroll
-      for (int v1 = 0; v1 < P; v1++) y[v1] = T1[rr][(k0 * P + v1) * P + v2];
-      dft15<1, P>(y);
+      for (int v1 = 0; v1 < P; v1++) v[v1] = T1[j][(k0 * P + v1) * P + v2];
+      dftInverse<L, R>(v, y, cw, sw);
 #pragma unroll
-      for (int k1 = 0; k1 < L; k1++) T2[rr][(k0 * L + k1) * P + v2] = y[k1];
+      for (int k1 = 0; k1 < L; k1++) T2[j][(k0 * L + k1) * P + v2] = y[k1];
     }
     __syncthreads();
-    for (int x = tid; x < NR * L * L; x += TB) {
-      const int rr = x / (L * L), z = x - rr * (L * L);
-      R2 y[P];
+    for (int x = tid; x < NT * L * L; x += TB) {
+      const int j = x / (L * L), z = x - j * (L * L);
+      R2 v[P], y[L];
 #pragma unroll
-      for (int v2 = 0; v2 < P; v2++) y[v2] = T2[rr][z * P + v2];
-      dft15<1, P>(y);
-      R2* Lr = Lout + rr * lStride + (size_t)t * LL + z * L;
+      for (int v2 = 0; v2 < P; v2++) v[v2] = T2[j][z * P + v2];
+      dftInverse<L, R>(v, y, cw, sw);
+      R2* Lr = Lout + (r0 + j) * lStride + (size_t)t * LL + z * L;
 #pragma unroll
       for (int k2 = 0; k2 < L; k2++) Lr[k2] = c2<R>(y[k2].x * inv, y[k2].y * inv);
-    }
-    return;
-  }
-  __syncthreads();  // twiddles in LDS
-#pragma unroll
-  for (int rr = 0; rr < NR; rr++) {
-    R2* Lr = Lout + rr * lStride + (size_t)t * LL;
-    if (rr > 0) __syncthreads();  // T1 / T2 of the previous right-hand side consumed
-    // axis 0 in registers: T1[k0 * P^2 + col] = sum_w0 J[w0, col] e^{+2 pi i w0 k0 / P}
-    if (tid < P2) {
-#pragma unroll
-      for (int k0 = 0; k0 < L; k0++) {
-        R2 s = c2<R>(0, 0);
-#pragma unroll
-        for (int m = 0; m < P; m++) {
-          const int q = (m * k0) % P;
-          const R2 v = acc[m][rr];
-          s.x += v.x * wc[q] - v.y * ws[q];
-          s.y += v.y * wc[q] + v.x * ws[q];
-        }
-        T1[0][k0 * P2 + tid] = s;
-      }
-    }
-    __syncthreads();
-    // axis 1: T2[(k0*L + k1)*P + w2], k1 < L
-    for (int x = tid; x < L * L * P; x += TB) {
-      const int v2 = x % P, k1 = (x / P) % L, k0 = x / (L * P);
-      R2 s = c2<R>(0, 0);
-#pragma unroll
-      for (int v1 = 0; v1 < P; v1++) {
-        const int q = (v1 * k1) % P;
-        const R2 v = T1[0][(k0 * P + v1) * P + v2];
-        s.x += v.x * wc[q] - v.y * ws[q];
-        s.y += v.y * wc[q] + v.x * ws[q];
-      }
-      T2[0][x] = s;
-    }
-    __syncthreads();
-    // axis 2 and scaling: L[(k0*L + k1)*L + k2]
-    for (int x = tid; x < LL; x += TB) {
-      const int k2 = x % L, r = x / L;
-      R2 s = c2<R>(0, 0);
-#pragma unroll
-      for (int v2 = 0; v2 < P; v2++) {
-        const int q = (v2 * k2) % P;
-        const R2 v = T2[0][r * P + v2];
-        s.x += v.x * wc[q] - v.y * ws[q];
-        s.y += v.y * wc[q] + v.x * ws[q];
-      }
-      Lr[x] = c2<R>(s.x * inv, s.y * inv);
     }
   }
 }
