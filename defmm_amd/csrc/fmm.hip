@@ -698,6 +698,22 @@ __global__ __launch_bounds__(256) void k_m2f(const int* __restrict__ m2fSlot,
 // in h to the axis-order index s (permutations.hpp:87-120).
 static const int kVariantOfSigma[8] = {0, 1, 0, 2, 3, 0, 4, 5};
 
+// Workgroups are dealt to the 8 XCDs in turn.  Each XCD gets a contiguous part
+// of the (level, direction, cell) group order, so that its L2 sees the groups
+// that share source rows; the parts hold equal shares of the rows to load
+// (m2lParts), not of the groups: equal counts gave the XCDs with the dense
+// levels up to 1.7 times the mean (20,000-point cube at 32 wavelengths), and
+// the others idled.  Block b takes item at[b mod 8] + b / 8, if it is in the
+// part (-1 otherwise).
+struct XcdParts {
+  int at[9];
+};
+__device__ __forceinline__ int partItem(const XcdParts& p, int b) {
+  const int x = b & 7;
+  const int i = p.at[x] + (b >> 3);
+  return i < p.at[x + 1] ? i : -1;
+}
+
 // M2L block shape for order L: NW frequencies per thread (at most 3 where a
 // block of <= 1024 threads covers PP, fewer when 256 threads suffice), TB
 // threads, G target slots per group.  A thread keeps NW F values, G x NW
@@ -837,21 +853,15 @@ __attribute__((amdgpu_waves_per_eu(m2lWavesPerEU<R, L, NR>(), 8))) void k_m2l(
     const int* __restrict__ gSrcF, const int* __restrict__ gMask, const int* __restrict__ gCode,
     const typename C2T<R>::T* __restrict__ F, size_t fStride,
     const typename C2T<R>::T* __restrict__ U, typename C2T<R>::T* __restrict__ Lout,
-    size_t lStride, const R* __restrict__ twc, const R* __restrict__ tws, int nItems) {
+    size_t lStride, const R* __restrict__ twc, const R* __restrict__ tws, XcdParts parts) {
   typedef typename C2T<R>::T R2;
   constexpr int P = 2 * L - 1, LL = L * L * L, PP = P * P * P;
   constexpr int NW = M2LShapeN<L, NR>::NW, TB = M2LShapeN<L, NR>::TB, G = M2LShapeN<L, NR>::G;
   constexpr int NU = G * NR, NB = f2lBatch(NU);
   __shared__ R2 J[NB * PP], T1[NB * L * P * P];
   const int tid = threadIdx.x;
-  // Workgroups are dealt to the 8 XCDs round-robin; give each XCD a
-  // contiguous part of the (direction-major) group order so that its L2 sees
-  // the groups that share source rows.  A bijection of [0, n8), n8 = n
-  // rounded down to a multiple of 8, and the identity on the tail.
-  const int b = itemIndex();
-  if (b >= nItems) return;
-  const int n8 = nItems & ~7;
-  const int grp = b < n8 ? (b & 7) * (n8 >> 3) + (b >> 3) : b;
+  const int grp = partItem(parts, itemIndex());
+  if (grp < 0) return;
   // frequencies of this thread, clamped to PP - 1: every load is in bounds
   // and unconditional, and the accumulators of w >= PP are never stored
   unsigned wl[NW];
@@ -976,7 +986,7 @@ __global__ __launch_bounds__(M2LShape<L>::TB) void k_m2l_col(
     const int* __restrict__ gSrcF, const int* __restrict__ gMask, const int* __restrict__ gCode,
     const typename C2T<R>::T* __restrict__ F, size_t fStride,
     const typename C2T<R>::T* __restrict__ U, typename C2T<R>::T* __restrict__ Lout,
-    size_t lStride, const R* __restrict__ twc, const R* __restrict__ tws, int nItems) {
+    size_t lStride, const R* __restrict__ twc, const R* __restrict__ tws, XcdParts parts) {
   typedef typename C2T<R>::T R2;
   constexpr int P = 2 * L - 1, P2 = P * P, LL = L * L * L, PP = P * P * P;
   constexpr int TB = M2LShape<L>::TB;
@@ -986,11 +996,8 @@ __global__ __launch_bounds__(M2LShape<L>::TB) void k_m2l_col(
   constexpr int NT = P == 15 ? NR : 1;
   __shared__ R2 T1[NT][L * P2], T2[NT][L * L * P];
   const int tid = threadIdx.x;
-  const int b = itemIndex();
-  if (b >= nItems) return;
-  // XCD-contiguous group order, as in k_m2l
-  const int n8 = nItems & ~7;
-  const int grp = b < n8 ? (b & 7) * (n8 >> 3) + (b >> 3) : b;
+  const int grp = partItem(parts, itemIndex());
+  if (grp < 0) return;
   // threads beyond the cube's columns load a valid column and store nothing
   const int col = min(tid, P2 - 1);
   R2 acc[P][NR];
@@ -1077,7 +1084,7 @@ __global__ __launch_bounds__(M2LShape<L>::TB) void k_m2l_fly(const int* __restri
                                                  const typename C2T<R>::T* __restrict__ U,
                                                  typename C2T<R>::T* __restrict__ Lout,
                                                  const R* __restrict__ twc,
-                                                 const R* __restrict__ tws, int nItems) {
+                                                 const R* __restrict__ tws, XcdParts parts) {
   typedef typename C2T<R>::T R2;
   constexpr int P = 2 * L - 1, LL = L * L * L, PP = P * P * P;
   constexpr int NW = M2LShape<L>::NW, TB = M2LShape<L>::TB, G = M2LShape<L>::G;
@@ -1085,10 +1092,8 @@ __global__ __launch_bounds__(M2LShape<L>::TB) void k_m2l_fly(const int* __restri
   __shared__ R2 sM[LL], B1[NB], B2[NB], J[PP];
   __shared__ R wc[P], ws[P];
   const int tid = threadIdx.x;
-  const int b = itemIndex();
-  if (b >= nItems) return;
-  const int n8 = nItems & ~7;
-  const int grp = b < n8 ? (b & 7) * (n8 >> 3) + (b >> 3) : b;
+  const int grp = partItem(parts, itemIndex());
+  if (grp < 0) return;
   if (tid < P) {
     wc[tid] = twc[tid];
     ws[tid] = tws[tid];
@@ -1873,6 +1878,9 @@ struct Exec {
   // slot map and the group bounds (the mode-dependent lists are built from them)
   ListVec hGSrcF;
   std::vector<int> hM2fSlot, hGroupBeg;
+  // rows that the M2L groups before each load (F rows, table rows and a share
+  // for the inverse transforms)
+  std::vector<int64_t> hGroupCost;
   double2 *qio = nullptr, *pio = nullptr;
   double stageMs[DEFMM_NSTAGES] = {};
   // host copies needed to re-upload the typed buffers in another precision
@@ -2522,6 +2530,15 @@ static int upload(Exec& X, Plan& pl) {
     X.st.m2l_table_rows = (int64_t)X.hRowKey.size();
     CKR(X.upv(X.gCode, dc));
   }
+  {
+    X.hGroupCost.assign(pl.m2lGroupBeg.size(), 0);
+    for (int g = 0; g < X.nGroups; g++) {
+      int64_t c = 4;
+      for (int e = pl.m2lGroupBeg[g]; e < pl.m2lGroupBeg[g + 1]; e++)
+        c += 1 + __builtin_popcount((unsigned)pl.m2lGMask[e]);
+      X.hGroupCost[g + 1] = X.hGroupCost[g] + c;
+    }
+  }
   X.hGSrcF.swap(pl.m2lGSrcF);
   X.hM2fSlot = pl.m2fSlot;
   X.hGroupBeg = pl.m2lGroupBeg;
@@ -2605,23 +2622,41 @@ static inline unsigned nblk(int64_t n, int b) { return (unsigned)((n + b - 1) / 
 
 // Launchers of the NR-wide kernels: the widest NR in {8, 4, 2, 1} that is
 // <= n and allowed, for right-hand sides r0 .. r0 + NR - 1.
+// Groups g0 .. g0 + ng - 1 (counted from g0) in 8 contiguous parts of equal
+// cost; grid: 8 times the largest part.
+static XcdParts m2lParts(const Exec& X, int g0, int ng, int64_t& grid) {
+  XcdParts p;
+  const auto first = X.hGroupCost.begin() + g0;
+  const int64_t c0 = *first, total = first[ng] - c0;
+  p.at[0] = 0;
+  p.at[8] = ng;
+  for (int x = 1; x < 8; x++)
+    p.at[x] = (int)(std::lower_bound(first, first + ng, c0 + total * x / 8) - first);
+  grid = 0;
+  for (int x = 0; x < 8; x++) grid = std::max<int64_t>(grid, p.at[x + 1] - p.at[x]);
+  grid *= 8;
+  return p;
+}
+
 template <typename R, int L, int NR>
 static void launchM2L(Exec& X, hipStream_t s, int g0, int ng, const typename C2T<R>::T* F,
                       typename C2T<R>::T* Lb, const OpConsts<R>& oc) {
   typedef typename C2T<R>::T R2;
   constexpr int G = M2LShapeN<L, NR>::G;
+  int64_t grid = 0;
+  const XcdParts parts = m2lParts(X, g0, ng, grid);
   if constexpr (M2LShape<L>::kColumns)
-    hipLaunchKernelGGL((k_m2l_col<R, L, NR>), itemGrid(ng), dim3(M2LShape<L>::TB), 0, s,
+    hipLaunchKernelGGL((k_m2l_col<R, L, NR>), itemGrid(grid), dim3(M2LShape<L>::TB), 0, s,
                        X.gBeg + g0, X.gTarget + (size_t)g0 * G, X.gSrc, X.gMask, X.gCode, F,
-                       X.fStride, (const R2*)X.U, Lb, X.lStride, oc.twc, oc.tws, ng);
+                       X.fStride, (const R2*)X.U, Lb, X.lStride, oc.twc, oc.tws, parts);
   else if (X.m2lSliced)
-    hipLaunchKernelGGL((k_m2l<R, L, NR, true>), itemGrid(ng), dim3(M2LShapeN<L, NR>::TB), 0, s,
+    hipLaunchKernelGGL((k_m2l<R, L, NR, true>), itemGrid(grid), dim3(M2LShapeN<L, NR>::TB), 0, s,
                        X.gBeg + g0, X.gTarget + (size_t)g0 * G, X.gSrc, X.gMask, X.gCode, F,
-                       X.fStride, (const R2*)X.U, Lb, X.lStride, oc.twc, oc.tws, ng);
+                       X.fStride, (const R2*)X.U, Lb, X.lStride, oc.twc, oc.tws, parts);
   else
-    hipLaunchKernelGGL((k_m2l<R, L, NR, false>), itemGrid(ng), dim3(M2LShapeN<L, NR>::TB), 0, s,
+    hipLaunchKernelGGL((k_m2l<R, L, NR, false>), itemGrid(grid), dim3(M2LShapeN<L, NR>::TB), 0, s,
                        X.gBeg + g0, X.gTarget + (size_t)g0 * G, X.gSrc, X.gMask, X.gCode, F,
-                       X.fStride, (const R2*)X.U, Lb, X.lStride, oc.twc, oc.tws, ng);
+                       X.fStride, (const R2*)X.U, Lb, X.lStride, oc.twc, oc.tws, parts);
 }
 
 // Right-hand sides of the next M2L launch when n are left.
@@ -2785,10 +2820,12 @@ static int runTyped(Exec& X, const double2* qin, double2* pout, int parts, int n
         r0 += m2lChunk<R, L>(X, s, 0, X.nGroups, r0, nrhs - r0, oc, Fr(r0));
     } else if (X.m2lMode == DEFMM_M2L_ON_THE_FLY) {
       if constexpr (!M2LShape<L>::kColumns) {
+        int64_t grid = 0;
+        const XcdParts all = m2lParts(X, 0, X.nGroups, grid);
         for (int r = 0; r < nrhs; r++)
-          hipLaunchKernelGGL((k_m2l_fly<R, L>), itemGrid(X.nGroups), dim3(M2LShape<L>::TB), 0,
-                             s, X.gBeg, X.gTarget, X.gSrc, X.gMask, X.gCode, (const R2*)Mr(r),
-                             (const R2*)X.U, Lr(r), oc.twc, oc.tws, X.nGroups);
+          hipLaunchKernelGGL((k_m2l_fly<R, L>), itemGrid(grid), dim3(M2LShape<L>::TB), 0, s,
+                             X.gBeg, X.gTarget, X.gSrc, X.gMask, X.gCode, (const R2*)Mr(r),
+                             (const R2*)X.U, Lr(r), oc.twc, oc.tws, all);
       } else {
         g_err = "the on-the-fly M2L variant supports orders up to 7";
         return ERR_ARG;
