@@ -22,6 +22,7 @@
 #include "grid.hpp"
 #include "dft.hpp"
 #include "kernels.hpp"
+#include "leaf_slots.hpp"
 #include "p2p.hpp"
 #include "plan.hpp"
 #include "xfer.hpp"
@@ -1831,6 +1832,19 @@ struct Exec {
   // points, and the vector-unit items of the larger leaves
   int2 *p2mMfmaItems = nullptr, *p2mBigItems = nullptr;
   int np2mMfma = 0, np2mBig = 0;
+  // matrix-core P2M of one right-hand side (leaf_slots.hpp): (leaf, first
+  // slot) of every leaf with several slots, and of those beyond 64 points
+  int2 *p2mSlotItems = nullptr, *p2mBigSlotItems = nullptr;
+  int np2mSlot = 0, np2mBigSlot = 0;
+  // and L2P: work items, tiles that several items share, partial sums
+  L2PItem* l2pItems = nullptr;
+  L2PTile* l2pShared = nullptr;
+  void* l2pPartial = nullptr;
+  int nl2pItems = 0, nl2pShared = 0;
+  struct LeafSlots {
+    int cell, n, ns, pbeg;
+  };
+  std::vector<LeafSlots> hL2PLeaf;
   bool p2mMfma = true;       // float P2M in chunks of 16 right-hand sides on the matrix cores
   bool m2lSliced = false;    // grouped M2L sweeps its entries once per frequency slice
   // (target leaf, first point) of the matrix-core L2P's point tiles, per
@@ -1919,6 +1933,9 @@ struct Exec {
     gSrc = bRows = nullptr;
     partial = qio = pio = nullptr;
     phaseTab = nullptr;
+    l2pItems = nullptr;
+    l2pShared = nullptr;
+    l2pPartial = nullptr;
   }
   // wait until the last execution, on whatever stream, has finished
   int quiesce() {
@@ -2191,6 +2208,41 @@ static int uploadTyped(Exec& X) {
     CKR(X.upv(d, t));
     X.phaseTab = d;
   }
+  {
+    // L2P items: tiles of at most TP points, the slots in equal ranges of at
+    // most `per` (multiples of 16); half as many where that leaves the chip
+    // idle
+    const int TP = l2pSlotTileAt(L, (int)sizeof(R));
+    std::vector<L2PItem> items;
+    std::vector<L2PTile> shared;
+    for (int per = kL2PSlots;; per /= 2) {
+      items.clear();
+      shared.clear();
+      int out = 0;
+      for (const auto& lf : X.hL2PLeaf) {
+        const int tiles = (lf.n + TP - 1) / TP, nt = (lf.n + tiles - 1) / tiles;
+        const int parts = (lf.ns + per - 1) / per;
+        const int len = ((lf.ns + parts - 1) / parts + kSlotCols - 1) / kSlotCols * kSlotCols;
+        for (int i0 = 0; i0 < lf.n; i0 += nt) {
+          const int np = std::min(nt, lf.n - i0), first = out;
+          for (int k0 = 0; k0 < lf.ns; k0 += len)
+            items.push_back({lf.cell, i0, np, k0, std::min(k0 + len, lf.ns),
+                             len < lf.ns ? out++ : -1});
+          if (out > first) shared.push_back({lf.pbeg + i0, np, first, out - first});
+        }
+      }
+      if (items.size() >= 2048 || per <= 64) {
+        void* d = nullptr;
+        CKR(X.alloc(d, (size_t)out * 32 * sizeof(R2)));
+        X.l2pPartial = d;
+        break;
+      }
+    }
+    CKR(X.upv(X.l2pItems, items));
+    X.nl2pItems = (int)items.size();
+    CKR(X.upv(X.l2pShared, shared));
+    X.nl2pShared = (int)shared.size();
+  }
   // right-hand side r of every store at base + r * stride
   const size_t nr = (size_t)X.nr;
   if (X.m2lMode == DEFMM_M2L_STORED) {
@@ -2418,27 +2470,50 @@ static int upload(Exec& X, Plan& pl) {
   CKR(X.upv(X.perm, pl.perm));
   CKR(X.upv(X.p2m, pl.p2mCell)); X.np2m = (int)pl.p2mCell.size();
   {
-    // P2M work items: every pass of p2mSlotsPerPass(L) slots of a leaf
+    // P2M work items: leaves with several slots on the matrix cores, the
+    // others in passes of p2mSlotsPerPass(L) slots
     const int C = p2mSlotsPerPass(pl.L);
-    std::vector<int2> it;
-    for (int c : pl.p2mCell)
-      for (int k0 = 0; k0 < std::max(1, pl.S.nslot[c]); k0 += C) it.push_back(make_int2(c, k0));
-    CKR(X.upv(X.p2mItems, it));
-    X.np2mItems = (int)it.size();
-    std::vector<int2> mf, big;
+    std::vector<int2> it, slots, mf, big, bigSlots;
     for (int c : pl.p2mCell) {
       const int nsl = std::max(1, pl.S.nslot[c]);
-      if (pl.S.nprt[c] <= kP2MMfmaPoints)
+      const bool small = pl.S.nprt[c] <= kP2MMfmaPoints;
+      if (nsl >= kP2MSlotsMin) {
+        for (int k0 = 0; k0 < nsl; k0 += kSlotCols) {
+          slots.push_back(make_int2(c, k0));
+          if (!small) bigSlots.push_back(make_int2(c, k0));
+        }
+      } else {
+        for (int k0 = 0; k0 < nsl; k0 += C) {
+          it.push_back(make_int2(c, k0));
+          if (!small) big.push_back(make_int2(c, k0));
+        }
+      }
+      if (small)
         for (int k0 = 0; k0 < nsl; k0 += kP2MMfmaSlots) mf.push_back(make_int2(c, k0));
-      else
-        for (int k0 = 0; k0 < nsl; k0 += C) big.push_back(make_int2(c, k0));
     }
+    CKR(X.upv(X.p2mItems, it));
+    X.np2mItems = (int)it.size();
+    CKR(X.upv(X.p2mSlotItems, slots));
+    X.np2mSlot = (int)slots.size();
     CKR(X.upv(X.p2mMfmaItems, mf));
     X.np2mMfma = (int)mf.size();
     CKR(X.upv(X.p2mBigItems, big));
     X.np2mBig = (int)big.size();
+    CKR(X.upv(X.p2mBigSlotItems, bigSlots));
+    X.np2mBigSlot = (int)bigSlots.size();
   }
-  CKR(X.upv(X.l2p, pl.l2pCell)); X.nl2p = (int)pl.l2pCell.size();
+  {
+    // L2P leaves of few slots (k_l2p); the others are cut into items at the
+    // typed upload (their tiles depend on the precision)
+    std::vector<int> few;
+    for (int c : pl.l2pCell) {
+      const int ns = pl.T.nslot[c];
+      if (ns >= l2pSlotsMin(pl.l2pCell.size())) X.hL2PLeaf.push_back({c, pl.T.nprt[c], ns, pl.T.pbeg[c]});
+      else few.push_back(c);
+    }
+    CKR(X.upv(X.l2p, few));
+    X.nl2p = (int)few.size();
+  }
   {
     // tiles of the matrix-core L2P: 32 points up to L^3 = 512, else 16
     const int tp = pl.LL <= 512 ? 32 : 16;
@@ -2768,7 +2843,17 @@ static int runTyped(Exec& X, const double2* qin, double2* pout, int parts, int n
   mark(1);
   const bool far = (parts & 2) != 0, near = (parts & 1) != 0;
 
-  if (far && X.np2mItems)
+  // P2M of one right-hand side: matrix-core items, then vector-unit items
+  auto launchP2M = [&](const int2* slots, int nSlots, const int2* few, int nFew, int r) {
+    if (nSlots)
+      hipLaunchKernelGGL((k_p2m_slots<R, L>), itemGrid(nSlots), dim3(64), 0, s, slots, X.S, X.lv,
+                         X.sx, X.sy, X.sz, (const R2*)qr(r), X.dirs, sig2, oc, X.kappa, Mr(r),
+                         nSlots);
+    if (nFew)
+      hipLaunchKernelGGL((k_p2m<R, L>), itemGrid(nFew), dim3(128), 0, s, few, X.S, X.lv, X.sx,
+                         X.sy, X.sz, (const R2*)qr(r), X.dirs, sig2, oc, X.kappa, Mr(r), nFew);
+  };
+  if (far)
     for (int r = 0; r < nrhs;) {
       if constexpr (sizeof(R) == 4) {
         if (nrhs - r >= kP2MMfmaNR && X.p2mMfma) {
@@ -2779,18 +2864,14 @@ static int runTyped(Exec& X, const double2* qin, double2* pout, int parts, int n
                                X.p2mMfmaItems, X.S, X.lv, X.sx, X.sy, X.sz,
                                (const float2*)qr(r), (size_t)ns, X.dirs, (const float2*)sig2, oc,
                                X.kappa, (float2*)Mr(r), X.mStride, X.np2mMfma);
-          if (X.np2mBig)
+          if (X.np2mBig || X.np2mBigSlot)
             for (int rr = r; rr < r + kP2MMfmaNR; rr++)
-              hipLaunchKernelGGL((k_p2m<R, L>), itemGrid(X.np2mBig), dim3(128), 0, s,
-                                 X.p2mBigItems, X.S, X.lv, X.sx, X.sy, X.sz, (const R2*)qr(rr),
-                                 X.dirs, sig2, oc, X.kappa, Mr(rr), X.np2mBig);
+              launchP2M(X.p2mBigSlotItems, X.np2mBigSlot, X.p2mBigItems, X.np2mBig, rr);
           r += kP2MMfmaNR;
           continue;
         }
       }
-      hipLaunchKernelGGL((k_p2m<R, L>), itemGrid(X.np2mItems), dim3(128), 0, s, X.p2mItems, X.S,
-                         X.lv, X.sx, X.sy, X.sz, (const R2*)qr(r), X.dirs, sig2, oc, X.kappa,
-                         Mr(r), X.np2mItems);
+      launchP2M(X.p2mSlotItems, X.np2mSlot, X.p2mItems, X.np2mItems, r);
       r++;
     }
   mark(2);
@@ -2859,7 +2940,7 @@ static int runTyped(Exec& X, const double2* qin, double2* pout, int parts, int n
       launchTrans<R, L>(t, (const R2*)Lr(0), Lr(0), sig2, sig, oc.B[0], oc.B[1], 1, X.lStride,
                         nrhs, s);
   mark(6);
-  if (far && X.nl2p)
+  if (far)
     for (int r = 0; r < nrhs;) {
       if constexpr (sizeof(R) == 4) {
         if (nrhs - r >= kL2PMfmaNR && X.l2pMfma) {
@@ -2871,9 +2952,18 @@ static int runTyped(Exec& X, const double2* qin, double2* pout, int parts, int n
           continue;
         }
       }
-      hipLaunchKernelGGL((k_l2p<R, L>), itemGrid(X.nl2p), dim3(256), 0, s, X.l2p, X.T, X.lv,
-                         X.tx, X.ty, X.tz, X.dirs, sig2, (const R2*)Lr(r), oc, X.kappa, pr(r),
-                         X.nl2p);
+      if (X.nl2pItems)
+        hipLaunchKernelGGL((k_l2p_slots<R, L>), itemGrid(X.nl2pItems), dim3(256), 0, s,
+                           X.l2pItems, X.T, X.lv, X.tx, X.ty, X.tz, X.dirs, sig2,
+                           (const R2*)Lr(r), oc, X.kappa, pr(r), (R2*)X.l2pPartial, X.nl2pItems);
+      if (X.nl2pShared)
+        hipLaunchKernelGGL(k_l2p_slots_reduce<R>, itemGrid(((int64_t)X.nl2pShared + 7) / 8),
+                           dim3(256), 0, s, X.l2pShared, (const R2*)X.l2pPartial, pr(r),
+                           X.nl2pShared);
+      if (X.nl2p)
+        hipLaunchKernelGGL((k_l2p<R, L>), itemGrid(X.nl2p), dim3(256), 0, s, X.l2p, X.T, X.lv,
+                           X.tx, X.ty, X.tz, X.dirs, sig2, (const R2*)Lr(r), oc, X.kappa, pr(r),
+                           X.nl2p);
       r++;
     }
   mark(7);
