@@ -590,6 +590,18 @@ __global__ __launch_bounds__(transLinesTB<L>()) void k_trans_lines(
 }
 
 
+// Elements from one Fourier row (of the F store or the M2L table store) to the
+// next: rows start at 16-byte addresses, for loads of 16 bytes per lane.  The
+// padding is never used.
+constexpr int rowStrideOf(int L, int elemBytes) {
+  const int PP = (2 * L - 1) * (2 * L - 1) * (2 * L - 1);
+  return elemBytes == 8 ? (PP + 1) / 2 * 2 : PP;
+}
+template <typename R, int L>
+constexpr int rowStride() {
+  return rowStrideOf(L, 2 * (int)sizeof(R));
+}
+
 // cos and sin of 2 pi m / P, m < L, of the plan's constants
 template <typename R, int L>
 __device__ __forceinline__ void loadTwiddles(const R* __restrict__ twc, const R* __restrict__ tws,
@@ -631,7 +643,7 @@ __global__ __launch_bounds__(256) void k_m2f(const int* __restrict__ m2fSlot,
                                              const R* __restrict__ tws, int nRows,
                                              size_t mStride, size_t fStride, int nrhs) {
   typedef typename C2T<R>::T R2;
-  constexpr int P = 2 * L - 1, LL = L * L * L, PP = P * P * P, NR = m2fRows<R, L>();
+  constexpr int P = 2 * L - 1, LL = L * L * L, NR = m2fRows<R, L>();
   __shared__ R2 T1[NR][L * L * P], T2[NR][L * P * P];
   const int tid = threadIdx.x;
   const int perRhs = (nRows + NR - 1) / NR;
@@ -674,7 +686,7 @@ __global__ __launch_bounds__(256) void k_m2f(const int* __restrict__ m2fSlot,
     R2 v[L], y[P];
 #pragma unroll
     for (int j = 0; j < L; j++) v[j] = T2[k][j * P * P + r];
-    R2* Fr = F + (size_t)(row0 + k) * PP + r;
+    R2* Fr = F + (size_t)(row0 + k) * rowStride<R, L>() + r;
     dftForward<L, R>(v, y, cw, sw);
 #pragma unroll
     for (int k0 = 0; k0 < P; k0++) Fr[k0 * P * P] = y[k0];
@@ -733,16 +745,25 @@ struct M2LShape {
       kColumns ? (P * P + 63) / 64 * 64 : ((PP + NW - 1) / NW + 63) / 64 * 64;
   static constexpr int G = m2lGroupSize(L);
 };
-// With NR right-hand sides per launch a thread holds G x NW x NR
-// accumulators in the same shape (measured faster than one frequency per
-// thread in 768-thread blocks: 144 vs 187 ms per right-hand side at 1M
-// points / 128 wavelengths / L = 5, float, two right-hand sides).
-template <int L, int NR>
+// Shape of the grouped kernel (L <= 7) for NR right-hand sides per launch.  A
+// thread owns NW units of V consecutive frequencies, 16 bytes: one double or
+// two float values (8-byte loads reach 18.6 TB/s from L2 on this chip, 16-byte
+// loads 31).  It holds G x NW x V x NR accumulators, at most 16 (double) or 32
+// (float) complex; of the NW that allow that, the largest with blocks of at
+// least two waves, none of them mostly idle.
+template <typename R, int L, int NR>
 struct M2LShapeN {
   static constexpr int PP = M2LShape<L>::PP;
-  static constexpr int NW = M2LShape<L>::NW;
-  static constexpr int TB = M2LShape<L>::TB;
   static constexpr int G = M2LShape<L>::G;
+  static constexpr int V = 16 / (2 * (int)sizeof(R));
+  static constexpr int UN = (PP + V - 1) / V;  // units of a row
+  static constexpr int tb(int nw) { return ((UN + nw - 1) / nw + 63) / 64 * 64; }
+  static constexpr bool fits(int nw) {
+    return G * nw * V * NR <= (sizeof(R) == 8 ? 16 : 32) && tb(nw) >= 128 &&
+           5 * UN >= 4 * nw * tb(nw);
+  }
+  static constexpr int NW = fits(3) ? 3 : fits(2) ? 2 : tb(1) <= 1024 ? 1 : M2LShape<L>::NW;
+  static constexpr int TB = tb(NW);
 };
 // Right-hand sides per M2L launch: at most 16 (double) or 32 (float)
 // complex accumulators per thread.
@@ -751,10 +772,11 @@ struct M2LShapeN {
 template <typename R, int L>
 constexpr int m2lMaxNR() {
   if (M2LShape<L>::kColumns) return sizeof(R) == 8 ? 1 : 2;
-  constexpr int NW = M2LShape<L>::NW;
-  constexpr int cap = (sizeof(R) == 8 ? 16 : 32) / (M2LShape<L>::G * NW);
-  constexpr int w = cap >= 8 ? 8 : cap >= 4 ? 4 : cap >= 2 ? 2 : 1;
-  return (sizeof(R) == 8 && L >= 7) ? 1 : (L == 7 && w > 2) ? 2 : w;
+  if (sizeof(R) == 8) {
+    constexpr int cap = 16 / (M2LShape<L>::G * M2LShape<L>::NW);
+    return L >= 7 ? 1 : cap >= 4 ? 4 : cap >= 2 ? 2 : 1;
+  }
+  return L <= 4 ? 4 : 2;
 }
 static int m2lMaxNRAt(int prec, int L) {
   switch (L) {
@@ -765,15 +787,6 @@ static int m2lMaxNRAt(int prec, int L) {
 #undef DFM_NR_CASE
     default: return 1;
   }
-}
-
-// Waves per SIMD the compiler is asked to fit: at L = 7 (768-thread blocks)
-// float with two right-hand sides took 105 VGPRs, one block per CU; 6 waves
-// per SIMD (two blocks) fit without spilling in groups of 3 targets (in
-// double they spill, so double keeps one block per CU).
-template <typename R, int L, int NR>
-constexpr int m2lWavesPerEU() {
-  return (L == 7 && sizeof(R) == 4) ? 6 : 1;
 }
 
 // F2L (F2L.hpp:35-46, circulant.hpp:108-118) of NB Fourier-domain expansions
@@ -833,9 +846,9 @@ __device__ __forceinline__ void f2lLines(typename C2T<R>::T* buf, typename C2T<R
 // lines) without more LDS than the occupancy that the registers allow.
 constexpr int f2lBatch(int units) { return units < 2 ? units : 2; }
 
-template <int PP>
+template <int RS>
 __device__ __forceinline__ size_t tableRow(int code) {
-  return (size_t)(code >> 3) * PP;
+  return (size_t)(code >> 3) * RS;
 }
 
 
@@ -848,8 +861,7 @@ __device__ __forceinline__ size_t tableRow(int code) {
 // accumulator sums the same terms in the same order with the same fused
 // multiply-adds (cmacFma): results are identical.
 template <typename R, int L, int NR, bool SL>
-__global__ __launch_bounds__((M2LShapeN<L, NR>::TB))
-__attribute__((amdgpu_waves_per_eu(m2lWavesPerEU<R, L, NR>(), 8))) void k_m2l(
+__global__ __launch_bounds__((M2LShapeN<R, L, NR>::TB)) void k_m2l(
     const int* __restrict__ groupBeg, const int* __restrict__ groupTarget,
     const int* __restrict__ gSrcF, const int* __restrict__ gMask, const int* __restrict__ gCode,
     const typename C2T<R>::T* __restrict__ F, size_t fStride,
@@ -857,49 +869,62 @@ __attribute__((amdgpu_waves_per_eu(m2lWavesPerEU<R, L, NR>(), 8))) void k_m2l(
     size_t lStride, const R* __restrict__ twc, const R* __restrict__ tws, XcdParts parts) {
   typedef typename C2T<R>::T R2;
   constexpr int P = 2 * L - 1, LL = L * L * L, PP = P * P * P;
-  constexpr int NW = M2LShapeN<L, NR>::NW, TB = M2LShapeN<L, NR>::TB, G = M2LShapeN<L, NR>::G;
+  typedef M2LShapeN<R, L, NR> Sh;
+  constexpr int NW = Sh::NW, TB = Sh::TB, G = Sh::G, V = Sh::V, RS = rowStride<R, L>();
+  struct alignas(16) Vec {
+    R2 v[V];
+  };
   constexpr int NU = G * NR, NB = f2lBatch(NU);
   __shared__ R2 J[NB * PP], T1[NB * L * P * P];
   const int tid = threadIdx.x;
   const int grp = partItem(parts, itemIndex());
   if (grp < 0) return;
-  // frequencies of this thread, clamped to PP - 1: every load is in bounds
-  // and unconditional, and the accumulators of w >= PP are never stored
+  // units of this thread, clamped to the row: every load is in bounds and
+  // unconditional, and the accumulators of w >= PP are never stored
   unsigned wl[NW];
 #pragma unroll
-  for (int m = 0; m < NW; m++) wl[m] = (unsigned)min(tid + TB * m, PP - 1);
-  R2 acc[G][NW][NR];
+  for (int m = 0; m < NW; m++) wl[m] = (unsigned)min(tid + TB * m, Sh::UN - 1);
+  R2 acc[G][NW][V][NR];
 #pragma unroll
   for (int g = 0; g < G; g++)
 #pragma unroll
     for (int m = 0; m < NW; m++)
 #pragma unroll
-      for (int r = 0; r < NR; r++) acc[g][m][r] = c2<R>(0, 0);
+      for (int v = 0; v < V; v++)
+#pragma unroll
+        for (int r = 0; r < NR; r++) acc[g][m][v][r] = c2<R>(0, 0);
   const int e0 = groupBeg[grp], e1 = groupBeg[grp + 1];
+  auto fRow = [&](int e, int r) {
+    return (const Vec*)(F + (size_t)r * fStride + (size_t)gSrcF[e] * RS);
+  };
+  auto uRow = [&](int e, int g) {
+    return (const Vec*)(U + tableRow<RS>(gCode[(size_t)e * G + g]));
+  };
   if constexpr (SL) {
     // one slice m at a time; entries e, e + 1 loaded together
-    auto ld = [&](int e, int m, R2 (&f)[NR], R2 (&u)[G], int& mask) {
-      const R2* Fr = F + (size_t)gSrcF[e] * PP + wl[m];
+    auto ld = [&](int e, int m, Vec (&f)[NR], Vec (&u)[G], int& mask) {
       mask = gMask[e];
 #pragma unroll
-      for (int r = 0; r < NR; r++) f[r] = Fr[r * fStride];
+      for (int r = 0; r < NR; r++) f[r] = fRow(e, r)[wl[m]];
 #pragma unroll
       for (int g = 0; g < G; g++)
-        if ((mask >> g) & 1) u[g] = U[tableRow<PP>(gCode[(size_t)e * G + g]) + wl[m]];
+        if ((mask >> g) & 1) u[g] = uRow(e, g)[wl[m]];
     };
-    auto mac = [&](int m, const R2 (&f)[NR], const R2 (&u)[G], int mask) {
+    auto mac = [&](int m, const Vec (&f)[NR], const Vec (&u)[G], int mask) {
 #pragma unroll
       for (int g = 0; g < G; g++) {
         if (!((mask >> g) & 1)) continue;
 #pragma unroll
-        for (int r = 0; r < NR; r++) cmacFma(acc[g][m][r], u[g], f[r]);
+        for (int v = 0; v < V; v++)
+#pragma unroll
+          for (int r = 0; r < NR; r++) cmacFma(acc[g][m][v][r], u[g].v[v], f[r].v[v]);
       }
     };
 #pragma unroll
     for (int m = 0; m < NW; m++) {
       int e = e0;
       for (; e + 1 < e1; e += 2) {
-        R2 fa[NR], ua[G], fb[NR], ub[G];
+        Vec fa[NR], ua[G], fb[NR], ub[G];
         int ma, mb;
         ld(e, m, fa, ua, ma);
         ld(e + 1, m, fb, ub, mb);
@@ -907,7 +932,7 @@ __attribute__((amdgpu_waves_per_eu(m2lWavesPerEU<R, L, NR>(), 8))) void k_m2l(
         mac(m, fb, ub, mb);
       }
       if (e < e1) {
-        R2 fa[NR], ua[G];
+        Vec fa[NR], ua[G];
         int ma;
         ld(e, m, fa, ua, ma);
         mac(m, fa, ua, ma);
@@ -915,22 +940,20 @@ __attribute__((amdgpu_waves_per_eu(m2lWavesPerEU<R, L, NR>(), 8))) void k_m2l(
     }
   } else
   for (int e = e0; e < e1; e++) {
-    const R2* Fr = F + (size_t)gSrcF[e] * PP;
     const int mask = gMask[e];
-    int code[G];
-#pragma unroll
-    for (int g = 0; g < G; g++) code[g] = gCode[(size_t)e * G + g];
     // issue all of the entry's loads before the first use
-    R2 f[NW][NR], u[G][NW];
+    Vec f[NW][NR], u[G][NW];
 #pragma unroll
-    for (int m = 0; m < NW; m++)
+    for (int r = 0; r < NR; r++) {
+      const Vec* Fr = fRow(e, r);
 #pragma unroll
-      for (int r = 0; r < NR; r++) f[m][r] = Fr[r * fStride + wl[m]];
+      for (int m = 0; m < NW; m++) f[m][r] = Fr[wl[m]];
+    }
 #pragma unroll
     for (int g = 0; g < G; g++) {
       // (u of a target absent from the entry is left unset and not read)
       if ((mask >> g) & 1) {
-        const R2* Ur = U + tableRow<PP>(code[g]);
+        const Vec* Ur = uRow(e, g);
 #pragma unroll
         for (int m = 0; m < NW; m++) u[g][m] = Ur[wl[m]];
       }
@@ -941,7 +964,9 @@ __attribute__((amdgpu_waves_per_eu(m2lWavesPerEU<R, L, NR>(), 8))) void k_m2l(
 #pragma unroll
       for (int m = 0; m < NW; m++)
 #pragma unroll
-        for (int r = 0; r < NR; r++) cmacFma(acc[g][m][r], u[g][m], f[m][r]);
+        for (int v = 0; v < V; v++)
+#pragma unroll
+          for (int r = 0; r < NR; r++) cmacFma(acc[g][m][v][r], u[g][m].v[v], f[m][r].v[v]);
     }
   }
   // F2L of the group's G x NR expansions, NB at a time
@@ -961,10 +986,12 @@ __attribute__((amdgpu_waves_per_eu(m2lWavesPerEU<R, L, NR>(), 8))) void k_m2l(
       const int t = groupTarget[(size_t)grp * G + g];
       if (t >= 0) dst[j] = Lout + rr * lStride + (size_t)t * LL;
 #pragma unroll
-      for (int m = 0; m < NW; m++) {
-        const int w = tid + TB * m;
-        if (w < PP) J[j * PP + w] = acc[g][m][rr];
-      }
+      for (int m = 0; m < NW; m++)
+#pragma unroll
+        for (int v = 0; v < V; v++) {
+          const int w = (tid + TB * m) * V + v;
+          if (w < PP) J[j * PP + w] = acc[g][m][v][rr];
+        }
     }
     __syncthreads();
     f2lLines<R, L, TB, NB>(J, T1, dst, inv, cw, sw, tid);
@@ -990,7 +1017,7 @@ __global__ __launch_bounds__(M2LShape<L>::TB) void k_m2l_col(
     size_t lStride, const R* __restrict__ twc, const R* __restrict__ tws, XcdParts parts) {
   typedef typename C2T<R>::T R2;
   constexpr int P = 2 * L - 1, P2 = P * P, LL = L * L * L, PP = P * P * P;
-  constexpr int TB = M2LShape<L>::TB;
+  constexpr int TB = M2LShape<L>::TB, RS = rowStride<R, L>();
   static_assert(M2LShape<L>::G == 1, "one target per group");
   // right-hand sides per F2L sweep: both at order 8, where their LDS still
   // lets two blocks share a CU
@@ -1008,8 +1035,8 @@ __global__ __launch_bounds__(M2LShape<L>::TB) void k_m2l_col(
     for (int r = 0; r < NR; r++) acc[m][r] = c2<R>(0, 0);
   const int e0 = groupBeg[grp], e1 = groupBeg[grp + 1];
   for (int e = e0; e < e1; e++) {
-    const R2* Fr = F + (size_t)gSrcF[e] * PP + col;
-    const R2* Ur = U + tableRow<PP>(gCode[e]) + col;
+    const R2* Fr = F + (size_t)gSrcF[e] * RS + col;
+    const R2* Ur = U + tableRow<RS>(gCode[e]) + col;
     // all of the entry's loads are issued before the first use
     R2 f[P][NR], u[P];
 #pragma unroll
@@ -1120,7 +1147,7 @@ __global__ __launch_bounds__(M2LShape<L>::TB) void k_m2l_fly(const int* __restri
     R2 u[G][NW];
 #pragma unroll
     for (int g = 0; g < G; g++) {
-      const R2* Ur = U + tableRow<PP>(gCode[(size_t)e * G + g]);
+      const R2* Ur = U + tableRow<rowStride<R, L>()>(gCode[(size_t)e * G + g]);
       if ((mask >> g) & 1) {
 #pragma unroll
         for (int m = 0; m < NW; m++) u[g][m] = Ur[wl[m]];
@@ -2089,7 +2116,8 @@ __constant__ int kTabAxisOrder[6][3] = {{0, 1, 2}, {1, 0, 2}, {1, 2, 0},
                                         {0, 2, 1}, {2, 0, 1}, {2, 1, 0}};
 template <typename R2>
 __global__ void k_table_rows(const int* __restrict__ keys, int64_t nrows,
-                             const R2* __restrict__ tab, int P, R2* __restrict__ rows) {
+                             const R2* __restrict__ tab, int P, int rowS,
+                             R2* __restrict__ rows) {
   const int64_t PP = (int64_t)P * P * P, n = nrows * PP;
   const int64_t stride = (int64_t)gridDim.x * blockDim.x;
   for (int64_t x = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; x < n; x += stride) {
@@ -2103,7 +2131,7 @@ __global__ void k_table_rows(const int* __restrict__ keys, int64_t nrows,
       if (((z >> j) & 1) && a[j]) a[j] = P - a[j];
     const int src = (a[kTabAxisOrder[s][0]] * P + a[kTabAxisOrder[s][1]]) * P +
                     a[kTabAxisOrder[s][2]];
-    rows[x] = tab[(int64_t)t * PP + src];
+    rows[k * rowS + i] = tab[(int64_t)t * PP + src];
   }
 }
 
@@ -2119,7 +2147,7 @@ static size_t partialElems(const Exec& X) {
 template <typename R>
 static int uploadTyped(Exec& X) {
   typedef typename C2T<R>::T R2;
-  const int L = X.L, P = X.P;
+  const int L = X.L, P = X.P, RS = rowStrideOf(L, sizeof(R2));
   X.typedPhase = true;
   {
     auto a = toR2<R>(X.hSig);
@@ -2141,10 +2169,10 @@ static int uploadTyped(Exec& X) {
         return ERR_STATE;
       }
     void* rows = nullptr;
-    CKR(X.alloc(rows, nrows * (size_t)PP * sizeof(R2)));
+    CKR(X.alloc(rows, nrows * (size_t)RS * sizeof(R2)));
     X.U = rows;
     if (ntab == 0) {
-      HIPCK(hipMemset(rows, 0, nrows * (size_t)PP * sizeof(R2)));
+      HIPCK(hipMemset(rows, 0, nrows * (size_t)RS * sizeof(R2)));
     } else {
       // the kernel tables and the keys are only needed here
       std::vector<R2> tab = toR2<R>(X.hTab);
@@ -2164,7 +2192,7 @@ static int uploadTyped(Exec& X) {
       } else {
         const int64_t n = (int64_t)nrows * PP;
         hipLaunchKernelGGL(k_table_rows<R2>, dim3(zeroGrid(n, 256)), dim3(256), 0, 0, dKeys,
-                           (int64_t)nrows, dTab, X.P, (R2*)rows);
+                           (int64_t)nrows, dTab, X.P, RS, (R2*)rows);
         if (hipGetLastError() != hipSuccess || hipDeviceSynchronize() != hipSuccess) {
           g_err = "M2L table rows kernel failed";
           rc = ERR_HIP;
@@ -2249,7 +2277,7 @@ static int uploadTyped(Exec& X) {
     // M is dead after M2F and every target slot's L is written by M2L or
     // zeroed: one buffer holds M, then L
     X.mStride = X.lStride = X.nMLslots * X.LL;
-    X.fStride = (size_t)std::max(1, X.nm2f) * X.PP;
+    X.fStride = (size_t)std::max(1, X.nm2f) * RS;
     CKR(X.alloc(X.ML, nr * X.mStride * sizeof(R2)));
     CKR(X.alloc(X.F, nr * X.fStride * sizeof(R2)));
     X.Lb = X.ML;
@@ -2271,7 +2299,7 @@ static int uploadTyped(Exec& X) {
       CKR(X.upv(X.gSrc, local));
       CKR(X.upv(X.bRows, rows));
       // the workspace holds the right-hand sides of one M2L launch
-      X.fStride = (size_t)X.wsRows * X.PP;
+      X.fStride = (size_t)X.wsRows * RS;
       const size_t nw = std::min(nr, (size_t)m2lMaxNRAt(X.prec, X.L));
       CKR(X.alloc(X.F, nw * X.fStride * sizeof(R2)));
     }
@@ -2306,7 +2334,7 @@ static int chooseM2LMode(Exec& X) {
     freeB = std::min(freeB, (size_t)std::max<int64_t>(0, X.memLimit - X.bytes));
   const size_t r2 = X.prec == DEFMM_FP64 ? 16 : 8;
   const size_t storedB =
-      (size_t)X.nr * (((size_t)X.nm2f * X.PP + X.nMLslots * X.LL) * r2 + ((size_t)X.ns + X.nt) * (r2 + 16)) +
+      (size_t)X.nr * (((size_t)X.nm2f * rowStrideOf(X.L, (int)r2) + X.nMLslots * X.LL) * r2 + ((size_t)X.ns + X.nt) * (r2 + 16)) +
       partialElems(X) * sizeof(double2) +
       (size_t)X.hGSrcF.size() * sizeof(int);
   X.m2lMode = (double)storedB < 0.9 * (double)freeB ? DEFMM_M2L_STORED : DEFMM_M2L_BATCHED;
@@ -2717,7 +2745,7 @@ template <typename R, int L, int NR>
 static void launchM2L(Exec& X, hipStream_t s, int g0, int ng, const typename C2T<R>::T* F,
                       typename C2T<R>::T* Lb, const OpConsts<R>& oc) {
   typedef typename C2T<R>::T R2;
-  constexpr int G = M2LShapeN<L, NR>::G;
+  constexpr int G = M2LShapeN<R, L, NR>::G;
   int64_t grid = 0;
   const XcdParts parts = m2lParts(X, g0, ng, grid);
   if constexpr (M2LShape<L>::kColumns)
@@ -2725,11 +2753,11 @@ static void launchM2L(Exec& X, hipStream_t s, int g0, int ng, const typename C2T
                        X.gBeg + g0, X.gTarget + (size_t)g0 * G, X.gSrc, X.gMask, X.gCode, F,
                        X.fStride, (const R2*)X.U, Lb, X.lStride, oc.twc, oc.tws, parts);
   else if (X.m2lSliced)
-    hipLaunchKernelGGL((k_m2l<R, L, NR, true>), itemGrid(grid), dim3(M2LShapeN<L, NR>::TB), 0, s,
+    hipLaunchKernelGGL((k_m2l<R, L, NR, true>), itemGrid(grid), dim3(M2LShapeN<R, L, NR>::TB), 0, s,
                        X.gBeg + g0, X.gTarget + (size_t)g0 * G, X.gSrc, X.gMask, X.gCode, F,
                        X.fStride, (const R2*)X.U, Lb, X.lStride, oc.twc, oc.tws, parts);
   else
-    hipLaunchKernelGGL((k_m2l<R, L, NR, false>), itemGrid(grid), dim3(M2LShapeN<L, NR>::TB), 0, s,
+    hipLaunchKernelGGL((k_m2l<R, L, NR, false>), itemGrid(grid), dim3(M2LShapeN<R, L, NR>::TB), 0, s,
                        X.gBeg + g0, X.gTarget + (size_t)g0 * G, X.gSrc, X.gMask, X.gCode, F,
                        X.fStride, (const R2*)X.U, Lb, X.lStride, oc.twc, oc.tws, parts);
 }
