@@ -44,43 +44,31 @@ static inline dim3 itemGrid(int64_t n) {
 // kernels
 // ----------------------------------------------------------------------------
 
-// fill a complex array with zeros (used instead of hipMemsetAsync so that the
-// sequence can be captured in a graph)
-// Grid-stride over n elements with a capped grid (zeroGrid), so that no
-// dispatch approaches 2^32 work-items whatever n is.
-template <typename R2>
-__global__ void k_zero(R2* a, int64_t n) {
-  const int64_t stride = (int64_t)gridDim.x * blockDim.x;
-  for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += stride) {
-    R2 z;
-    z.x = 0;
-    z.y = 0;
-    a[i] = z;
-  }
-}
-
-// Tree::loadRHS (tree.hpp:149-154): q_tree[i] = q_in[perm[i]]
+// Tree::loadRHS (tree.hpp:149-154): q_tree[i] = q_in[perm[i]], and the
+// potentials cleared, for the right-hand sides blockIdx.y
 template <typename R>
 __global__ void k_gather(const double2* __restrict__ qin, const int* __restrict__ perm,
-                         typename C2T<R>::T* __restrict__ q, int n) {
-  int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i < n) {
-    double2 v = qin[perm[i]];
-    q[i] = c2<R>((R)v.x, (R)v.y);
+                         typename C2T<R>::T* __restrict__ q, int ns,
+                         typename C2T<R>::T* __restrict__ p, int nt) {
+  const int i = blockIdx.x * blockDim.x + threadIdx.x;
+  const size_t r = blockIdx.y;
+  if (i < ns) {
+    const double2 v = qin[r * ns + perm[i]];
+    q[r * ns + i] = c2<R>((R)v.x, (R)v.y);
   }
+  if (i < nt) p[r * nt + i] = c2<R>(0, 0);
 }
 
-// Tree::writeLHS (tree.hpp:156-160): p_out[perm[i]] = p_tree[i]
+// Tree::writeLHS (tree.hpp:156-160): p_out[perm[i]] = p_tree[i], for the
+// right-hand sides blockIdx.y
 template <typename R>
 __global__ void k_scatter(const typename C2T<R>::T* __restrict__ p, const int* __restrict__ perm,
                           double2* __restrict__ pout, int n) {
-  int i = blockIdx.x * blockDim.x + threadIdx.x;
+  const int i = blockIdx.x * blockDim.x + threadIdx.x;
+  const size_t r = blockIdx.y;
   if (i < n) {
-    typename C2T<R>::T v = p[i];
-    double2 o;
-    o.x = (double)v.x;
-    o.y = (double)v.y;
-    pout[perm[i]] = o;
+    const typename C2T<R>::T v = p[r * n + i];
+    pout[r * n + perm[i]] = make_double2((double)v.x, (double)v.y);
   }
 }
 
@@ -1270,7 +1258,8 @@ __global__ __launch_bounds__(M2LShape<L>::TB) void k_m2l_fly(const int* __restri
 }
 
 // L = 0 for the target slots that receive no M2L (their L gets only L2L).
-// (grid-stride with a capped grid, as k_zero)
+// (grid-stride over n elements with a capped grid (zeroGrid), so that no
+// dispatch approaches 2^32 work-items whatever n is)
 template <typename R, int L>
 __global__ __launch_bounds__(256) void k_zero_slots(const int* __restrict__ slots, int n,
                                                     typename C2T<R>::T* __restrict__ Lout) {
@@ -2505,7 +2494,7 @@ static int upload(Exec& X, Plan& pl) {
     for (int c : pl.p2mCell) {
       const int nsl = std::max(1, pl.S.nslot[c]);
       const bool small = pl.S.nprt[c] <= kP2MMfmaPoints;
-      if (nsl >= kP2MSlotsMin) {
+      if (nsl >= p2mSlotsMin(pl.p2mCell.size())) {
         for (int k0 = 0; k0 < nsl; k0 += kSlotCols) {
           slots.push_back(make_int2(c, k0));
           if (!small) bigSlots.push_back(make_int2(c, k0));
@@ -2863,11 +2852,9 @@ static int runTyped(Exec& X, const double2* qin, double2* pout, int parts, int n
     if (!X.capturing) (void)hipEventRecord(X.ev[k], s);
   };
   mark(0);
-  hipLaunchKernelGGL(k_zero<R2>, dim3(zeroGrid((int64_t)nrhs * (int64_t)nt, 256)), dim3(256), 0,
-                     s, (R2*)X.p, (int64_t)nrhs * (int64_t)nt);
-  for (int r = 0; r < nrhs; r++)
-    hipLaunchKernelGGL(k_gather<R>, dim3(nblk(X.ns, 256)), dim3(256), 0, s, qin + r * ns,
-                       X.sperm, qr(r), (int)X.ns);
+  // (kernels clear memory, so that the sequence can be captured in a graph)
+  hipLaunchKernelGGL(k_gather<R>, dim3(nblk(std::max(X.ns, X.nt), 256), (unsigned)nrhs),
+                     dim3(256), 0, s, qin, X.sperm, qr(0), (int)X.ns, pr(0), (int)X.nt);
   mark(1);
   const bool far = (parts & 2) != 0, near = (parts & 1) != 0;
 
@@ -3014,9 +3001,8 @@ static int runTyped(Exec& X, const double2* qin, double2* pout, int parts, int n
     }
   }
   mark(8);
-  for (int r = 0; r < nrhs; r++)
-    hipLaunchKernelGGL(k_scatter<R>, dim3(nblk(X.nt, 256)), dim3(256), 0, s, (const R2*)pr(r),
-                       X.tperm, pout + r * nt, (int)X.nt);
+  hipLaunchKernelGGL(k_scatter<R>, dim3(nblk(X.nt, 256), (unsigned)nrhs), dim3(256), 0, s,
+                     (const R2*)pr(0), X.tperm, pout, (int)X.nt);
   mark(9);
   if (!X.capturing) X.evRecorded = true;
   HIPCK(hipGetLastError());
@@ -3219,7 +3205,11 @@ int defmm_plan_create(const double* src_xyz, int64_t n_src, const double* trg_xy
     if (rc == dfm::OK && hipEventCreateWithFlags(&h->x.done, hipEventDisableTiming) != hipSuccess)
       rc = DEFMM_EHIP;
     for (auto& e : h->x.ev)
-      if (rc == dfm::OK && hipEventCreate(&e) != hipSuccess) rc = DEFMM_EHIP;
+      // stage times only: without the system-scope fence a record costs the
+      // stream 1 us instead of 6 (10 a pass: 4,000 points 207 -> 189 us)
+      if (rc == dfm::OK &&
+          hipEventCreateWithFlags(&e, hipEventDisableSystemFence) != hipSuccess)
+        rc = DEFMM_EHIP;
   }
   if (rc != dfm::OK) {
     delete h;

@@ -23,10 +23,10 @@ constexpr int kSlotCols = 16;    // slots per matrix-core tile
 // slots a leaf (41,334 points, order 6, double) 0.28 against 0.49; P2M, whose
 // vector kernel is further behind, gains from 6 slots on (1.19 -> 0.91 ms).
 // Plans of few leaves leave SIMDs idle on either path, so rounding up costs
-// nothing there and splitting a leaf's slots over blocks pays (510 leaves,
-// order 10: L2P 0.61 -> 0.42 ms with the line at 6).
-constexpr int kP2MSlotsMin = 6;
-inline int l2pSlotsMin(size_t leaves) { return leaves < 2048 ? 6 : 24; }
+// nothing there, splitting a leaf's slots over blocks pays (510 leaves, order
+// 10: L2P 0.61 -> 0.42 ms with the line at 6), and one kernel does for all.
+inline int p2mSlotsMin(size_t leaves) { return leaves < 2048 ? 1 : 6; }
+inline int l2pSlotsMin(size_t leaves) { return leaves < 2048 ? 1 : 24; }
 constexpr int kL2PSlots = 128;   // slots per block of k_l2p_slots
 
 typedef double mfma_v4d __attribute__((ext_vector_type(4)));
