@@ -1551,222 +1551,6 @@ __global__ __launch_bounds__(256) void k_l2p_mfma(
   }
 }
 
-// P2P near field (P2P.hpp:42-79) on the matrix cores.  A work item is up to
-// 64 targets of one leaf against a run of its source list; it writes
-// per-target partial sums (double).
-struct P2PItem {
-  int leaf;  // index into the leaf list
-  int t0;    // first target of the chunk (leaf-relative)
-  int r;     // first source range
-  int off;   // offset into that range
-  int cnt;   // number of sources
-};
-
-// Kernel value G = exp(i kappa r) / (4 pi r) between a target and a source
-// (P2P.hpp:61-75), 0 when r^2 < 1e-16.
-// Small: kappa * r <= 2^20 for every pair (checked on the host), so the
-// double sine and cosine need no range check.
-template <typename R, bool Small>
-__device__ __forceinline__ void p2pKernel(double xt, double yt, double zt, double xs, double ys,
-                                          double zs, double kappa, R& co, R& si);
-template <>
-__device__ __forceinline__ void p2pKernel<float, true>(double xt, double yt, double zt,
-                                                       double xs, double ys, double zs,
-                                                       double kappa, float& co, float& si);
-template <>
-__device__ __forceinline__ void p2pKernel<float, false>(double xt, double yt, double zt,
-                                                        double xs, double ys, double zs,
-                                                        double kappa, float& co, float& si) {
-  const double x = xt - xs, y = yt - ys, z = zt - zs;
-  const double R2v = x * x + y * y + z * z;
-  // r to ~1e-14 relative: float reciprocal square root, one Newton step in double
-  const float y0 = (R2v < 1.e-16) ? 0.f : rsqrtf((float)R2v);
-  const double r0 = R2v * (double)y0;
-  const double r = fma(0.5 * (double)y0, fma(-r0, r0, R2v), r0);
-  const float K = y0 * 0.079577471545947667884f;
-  expi(kappa * r, co, si);
-  co *= K;
-  si *= K;
-}
-template <>
-__device__ __forceinline__ void p2pKernel<float, true>(double xt, double yt, double zt,
-                                                       double xs, double ys, double zs,
-                                                       double kappa, float& co, float& si) {
-  const double x = xt - xs, y = yt - ys, z = zt - zs;
-  const double R2v = x * x + y * y + z * z;
-  const float y0 = (R2v < 1.e-16) ? 0.f : rsqrtf((float)R2v);
-  const double r0 = R2v * (double)y0;
-  const double r = fma(0.5 * (double)y0, fma(-r0, r0, R2v), r0);
-  const float K = y0 * 0.079577471545947667884f;
-  sincosRedF(kappa * r, si, co);
-  co *= K;
-  si *= K;
-}
-
-// P2P for 16 right-hand sides per launch on the matrix cores (float, the
-// mixed-precision path).  An item's near-field sum is the product of the
-// kernel matrix G (targets x sources, complex, evaluated by the VALU one
-// element per lane, phase reduced in double) and the charge matrix
-// Q (sources x 16 right-hand sides):
-//   P_re += G_re Q_re - G_im Q_im,   P_im += G_re Q_im + G_im Q_re,
-// four V_MFMA_F32_16X16X4_F32 per 4 sources.  Operand layouts of that
-// instruction: A (16 x 4) lane l holds row l % 16, column l / 16; B (4 x 16)
-// lane l holds row l / 16, column l % 16; D (16 x 16) lane l holds column
-// l % 16, rows 4 (l / 16) + 0..3.  So lane l evaluates G for target
-// 16 w + l % 16 (wave w of the block's 4) and source 4 k + l / 16 of the
-// current K-step k, and ends holding right-hand side l % 16 of targets
-// 16 w + 4 (l / 16) + 0..3.  Sources are staged 64 at a time in LDS (the
-// charges as [source][right-hand side]); each 64-source tile's sums are added
-// to double accumulators and the item's partial sums go to
-// the layout k_p2p_reduce<float, 16> reads.
-constexpr int kP2PMfmaNR = 16;
-
-template <bool Small>
-__global__ __launch_bounds__(256) void k_p2p_mfma(
-    const P2PItem* __restrict__ items, const int* __restrict__ leafCell,
-    const int* __restrict__ tpbeg, const int* __restrict__ tnprt, const double* __restrict__ tx,
-    const double* __restrict__ ty, const double* __restrict__ tz, const double* __restrict__ sx,
-    const double* __restrict__ sy, const double* __restrict__ sz, const float2* __restrict__ q,
-    size_t qStride, const int* __restrict__ rb, const int* __restrict__ re, double kappa,
-    double2* __restrict__ partial, int nItems) {
-  __shared__ double lx[64], ly[64], lz[64];
-  __shared__ int lj[64];
-  __shared__ float2 lq[64][kP2PMfmaNR];
-  const int item = itemIndex();
-  if (item >= nItems) return;
-  const P2PItem it = items[item];
-  const int c = leafCell[it.leaf];
-  const int tb = tpbeg[c] + it.t0;
-  const int nt = min(64, tnprt[c] - it.t0);
-  const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
-  const int ti = wave * 16 + (lane & 15);  // target of this lane's A row
-  const bool tok = ti < nt;
-  const bool waveOn = wave * 16 < nt;      // uniform over the wave
-  double xt = 0., yt = 0., zt = 0.;
-  if (tok) {
-    xt = tx[tb + ti];
-    yt = ty[tb + ti];
-    zt = tz[tb + ti];
-  }
-  const int kq = lane >> 4, rq = lane & 15;
-  mfma_v4f dre = {0.f, 0.f, 0.f, 0.f}, dim = {0.f, 0.f, 0.f, 0.f};
-  double accr[4] = {0., 0., 0., 0.}, acci[4] = {0., 0., 0., 0.};
-  int r = it.r, off = it.off;
-  for (int pos = 0; pos < it.cnt; pos += 64) {
-    const int tileN = min(64, it.cnt - pos);
-    __syncthreads();
-    if (tid < 64) {
-      int j = -1;
-      if (tid < tileN) {
-        int rr = r, oo = off + tid;
-        int len = re[rr] - rb[rr];
-        while (oo >= len) {
-          oo -= len;
-          rr++;
-          len = re[rr] - rb[rr];
-        }
-        j = rb[rr] + oo;
-        lx[tid] = sx[j];
-        ly[tid] = sy[j];
-        lz[tid] = sz[j];
-      }
-      lj[tid] = j;
-    }
-    {
-      int adv = tileN;
-      while (adv > 0) {
-        const int rem = re[r] - rb[r] - off;
-        if (adv < rem) {
-          off += adv;
-          adv = 0;
-        } else {
-          adv -= rem;
-          r++;
-          off = 0;
-        }
-      }
-    }
-    __syncthreads();
-    for (int x = tid; x < 64 * kP2PMfmaNR; x += 256) {
-      const int sj = x / kP2PMfmaNR, rr = x % kP2PMfmaNR;
-      const int j = lj[sj];
-      lq[sj][rr] = j >= 0 ? q[rr * qStride + j] : make_float2(0.f, 0.f);
-    }
-    __syncthreads();
-    if (waveOn) {
-      for (int k = 0; k < 16; k++) {
-        const int j = 4 * k + kq;
-        float gr = 0.f, gi = 0.f;
-        if (tok && j < tileN) p2pKernel<float, Small>(xt, yt, zt, lx[j], ly[j], lz[j], kappa, gr, gi);
-        const float2 b = lq[j][rq];
-        dre = __builtin_amdgcn_mfma_f32_16x16x4f32(gr, b.x, dre, 0, 0, 0);
-        dre = __builtin_amdgcn_mfma_f32_16x16x4f32(-gi, b.y, dre, 0, 0, 0);
-        dim = __builtin_amdgcn_mfma_f32_16x16x4f32(gr, b.y, dim, 0, 0, 0);
-        dim = __builtin_amdgcn_mfma_f32_16x16x4f32(gi, b.x, dim, 0, 0, 0);
-      }
-#pragma unroll
-      for (int v = 0; v < 4; v++) {
-        accr[v] += (double)dre[v];
-        acci[v] += (double)dim[v];
-        dre[v] = 0.f;
-        dim[v] = 0.f;
-      }
-    }
-  }
-  if (waveOn)
-#pragma unroll
-    for (int v = 0; v < 4; v++) {
-      const int t = wave * 16 + 4 * kq + v;
-      if (t < nt)
-        partial[((size_t)item * kP2PMfmaNR + rq) * 64 + t] = make_double2(accr[v], acci[v]);
-    }
-}
-
-// Sum the partial results of a leaf's items into p (items of a leaf are
-// contiguous, ordered by target chunk).
-// NR right-hand sides (partial sums of item k, right-hand side r, target t at
-// partial[(k * NR + r) * 64 + t]); right-hand side r adds into p + r * pStride.
-template <typename R, int NR>
-__global__ __launch_bounds__(64) void k_p2p_reduce(const int* __restrict__ itemBeg,
-                                                   const P2PItem* __restrict__ items,
-                                                   const int* __restrict__ leafCell,
-                                                   const int* __restrict__ tpbeg,
-                                                   const int* __restrict__ tnprt,
-                                                   const double2* __restrict__ partial,
-                                                   typename C2T<R>::T* __restrict__ p,
-                                                   size_t pStride, int nItems) {
-  typedef typename C2T<R>::T R2;
-  const int leaf = itemIndex();
-  if (leaf >= nItems) return;
-  const int c = leafCell[leaf];
-  const int pb = tpbeg[c], n = tnprt[c];
-  const int ib = itemBeg[leaf], ie = itemBeg[leaf + 1];
-  for (int t0 = 0; t0 < n; t0 += 64) {
-    const int i = t0 + threadIdx.x;
-    double sr[NR], si[NR];
-#pragma unroll
-    for (int r = 0; r < NR; r++) sr[r] = si[r] = 0.;
-    for (int k = ib; k < ie; k++) {
-      if (items[k].t0 != t0) continue;
-#pragma unroll
-      for (int r = 0; r < NR; r++) {
-        const double2 v = partial[((size_t)k * NR + r) * 64 + threadIdx.x];
-        sr[r] += v.x;
-        si[r] += v.y;
-      }
-    }
-    if (i < n) {
-#pragma unroll
-      for (int r = 0; r < NR; r++) {
-        R2 o = p[r * pStride + pb + i];
-        o.x = (R)((double)o.x + sr[r]);
-        o.y = (R)((double)o.y + si[r]);
-        p[r * pStride + pb + i] = o;
-      }
-    }
-  }
-}
-
 // ----------------------------------------------------------------------------
 // executor
 // ----------------------------------------------------------------------------
@@ -1883,7 +1667,7 @@ struct Exec {
   P2PItem* items = nullptr;
   int nitems = 0;
   // items of the near field with a lane per source (p2p.hpp)
-  P2PLaneItem* laneItems = nullptr;
+  P2PItem* laneItems = nullptr;
   int nLaneItems = 0;
   int* laneItemBeg = nullptr;
   int p2pPhase = kPhaseLibrary;
@@ -1896,7 +1680,6 @@ struct Exec {
   void* Lb = nullptr;        // local expansions (aliases ML when F is stored)
   size_t mStride = 0, lStride = 0, fStride = 0;  // elements between right-hand sides
   int m2lMode = DEFMM_M2L_STORED;
-  int smallArg = 0;          // kappa * (largest point distance) <= 2^20
   bool p2pMfma = true;       // float P2P in chunks of 16 right-hand sides on the matrix cores
   bool m2lAuto = true;       // mode chosen by free memory (until set explicitly)
   int nr = 1;                // right-hand sides the expansion stores hold
@@ -2129,7 +1912,7 @@ __global__ void k_table_rows(const int* __restrict__ keys, int64_t nrows,
 static size_t partialElems(const Exec& X) {
   size_t n = (size_t)X.nLaneItems * std::min(X.nr, X.prec == DEFMM_MIXED ? 8 : 4) * kP2PTargets;
   if (X.prec == DEFMM_MIXED && X.nr >= kP2PMfmaNR)
-    n = std::max(n, (size_t)X.nitems * 64 * kP2PMfmaNR);
+    n = std::max(n, (size_t)X.nitems * kP2PMfmaTargets * kP2PMfmaNR);
   return std::max<size_t>(n, 1);
 }
 
@@ -2366,22 +2149,21 @@ static int reupload(Exec& X, int oldNr, int oldPrec, int oldMode, bool oldAuto, 
   return rc;
 }
 
-// Items of the near field with a lane per source: a leaf's targets in equal
-// chunks of at most kP2PTargets, its source list in equal runs (multiples of
-// 64) of at most `budget` sources.  8,192 sources a run amortise the final
-// sum over the wave; where that leaves fewer than 16,384 items (16 waves per
-// SIMD's share of the chip are needed to hide latency and even out the end)
-// the budget is halved, down to 512.
-static int buildLaneItems(Exec& X, const Plan& pl) {
+// Near-field items: a leaf's targets in chunks of at most tg (p2pChunk), its
+// source list in equal runs (multiples of 64) of at most `budget` sources.
+// 8,192 sources a run amortise a wave's start and final sums; where that
+// leaves fewer than 16,384 items (16 waves per SIMD's share of the chip are
+// needed to hide latency and even out the end) the budget is halved, down to
+// 512.
+static int buildP2PItems(const Plan& pl, int tg, std::vector<P2PItem>& items,
+                         std::vector<int>& beg) {
   const Tree& T = pl.T;
   const size_t nl = pl.p2pLeaf.size();
-  std::vector<P2PLaneItem> items;
-  std::vector<int> beg;
   std::vector<int64_t> total(nl, 0);
   for (size_t lf = 0; lf < nl; lf++)
     for (int r = pl.p2pBeg[lf]; r < pl.p2pBeg[lf + 1]; r++)
       total[lf] += pl.p2pSrcE[r] - pl.p2pSrcB[r];
-  auto chunksOf = [&](size_t lf) { return (T.nprt[pl.p2pLeaf[lf]] + kP2PTargets - 1) / kP2PTargets; };
+  auto chunksOf = [&](size_t lf) { return (T.nprt[pl.p2pLeaf[lf]] + tg - 1) / tg; };
   int64_t budget = 8192;
   for (;; budget /= 2) {
     int64_t n = 0;
@@ -2400,7 +2182,7 @@ static int buildLaneItems(Exec& X, const Plan& pl) {
     const int n = T.nprt[pl.p2pLeaf[lf]], chunks = chunksOf(lf);
     const int64_t runs = (total[lf] + budget - 1) / budget;
     if (runs == 0 || chunks == 0) continue;
-    const int chunk = (n + chunks - 1) / chunks;
+    const int chunk = p2pChunk(n, tg);
     const int64_t len = ((total[lf] + runs - 1) / runs + 63) / 64 * 64;
     int r = pl.p2pBeg[lf], off = 0;
     for (int64_t pos = 0; pos < total[lf]; pos += len) {
@@ -2413,16 +2195,13 @@ static int buildLaneItems(Exec& X, const Plan& pl) {
         items.push_back({(int)lf, t0, std::min(chunk, n - t0), r, off, cnt});
       off += cnt;
     }
-    // the reduction counts ceil(n / kP2PTargets) items per run
+    // the reduction counts ceil(n / tg) items per run
     if (((int)items.size() - beg.back()) % chunks != 0) {
       g_err = "internal: near-field items do not match the leaf's chunks";
       return ERR_STATE;
     }
   }
   beg.push_back((int)items.size());
-  X.nLaneItems = (int)items.size();
-  CKR(X.upv(X.laneItems, items));
-  CKR(X.upv(X.laneItemBeg, beg));
   return OK;
 }
 
@@ -2442,9 +2221,9 @@ static int upload(Exec& X, Plan& pl) {
       }
     double diag2 = 0.;
     for (int d = 0; d < 3; d++) diag2 += (hi[d] - lo[d]) * (hi[d] - lo[d]);
-    X.smallArg = std::fabs(pl.kappa) * std::sqrt(diag2) * (1. + 1e-12) <= 1048576.0 ? 1 : 0;
+    X.p2pPhase = phaseOf(X.kappa, std::fabs(pl.kappa) * std::sqrt(diag2) * (1. + 1e-12) <=
+                                      1048576.0);
   }
-  X.p2pPhase = phaseOf(X.kappa, X.smallArg != 0);
   X.phaseConsts = phaseConstsOf(X.kappa);
   X.st = pl.st;
   X.ns = (int64_t)pl.S.x.size();
@@ -2640,62 +2419,20 @@ static int upload(Exec& X, Plan& pl) {
   // is halved, down to 512.
   {
     std::vector<P2PItem> items;
-    std::vector<int> itemBeg;
-    const Tree& T = pl.T;
-    auto build = [&](int kBudget) {
-      items.clear();
-      itemBeg.clear();
-      for (size_t lf = 0; lf < pl.p2pLeaf.size(); lf++) {
-        itemBeg.push_back((int)items.size());
-        int c = pl.p2pLeaf[lf];
-        for (int t0 = 0; t0 < T.nprt[c]; t0 += 64) {
-          int r = pl.p2pBeg[lf], off = 0, cnt = 0, r0 = r, off0 = 0;
-          for (; r < pl.p2pBeg[lf + 1]; r++) {
-            int len = pl.p2pSrcE[r] - pl.p2pSrcB[r];
-            off = 0;
-            while (off < len) {
-              int take = std::min(len - off, kBudget - cnt);
-              if (cnt == 0) { r0 = r; off0 = off; }
-              cnt += take;
-              off += take;
-              if (cnt == kBudget) {
-                items.push_back({(int)lf, t0, r0, off0, cnt});
-                cnt = 0;
-              }
-            }
-          }
-          if (cnt) items.push_back({(int)lf, t0, r0, off0, cnt});
-        }
-      }
-      itemBeg.push_back((int)items.size());
-    };
-    for (int budget = 4096;; budget /= 2) {
-      build(budget);
-      if (items.size() >= 16384 || budget <= 512) break;
-    }
-    // the kernel walks ranges from (r, off) for cnt sources: they must stay
-    // inside the item's leaf list
-    for (const P2PItem& it : items) {
-      int rEnd = pl.p2pBeg[it.leaf + 1];
-      if (it.r < pl.p2pBeg[it.leaf] || it.r >= rEnd || it.cnt < 1 || it.t0 < 0 ||
-          it.t0 >= T.nprt[pl.p2pLeaf[it.leaf]]) {
-        g_err = "internal: P2P item out of range";
-        return ERR_STATE;
-      }
-      int64_t avail = -(int64_t)it.off;
-      for (int r = it.r; r < rEnd; r++) avail += pl.p2pSrcE[r] - pl.p2pSrcB[r];
-      if (it.off < 0 || it.off >= pl.p2pSrcE[it.r] - pl.p2pSrcB[it.r] || it.cnt > avail) {
-        g_err = "internal: P2P item exceeds its source list";
-        return ERR_STATE;
-      }
-    }
+    std::vector<int> beg;
+    CKR(buildP2PItems(pl, kP2PTargets, items, beg));
+    X.nLaneItems = (int)items.size();
+    CKR(X.upv(X.laneItems, items));
+    CKR(X.upv(X.laneItemBeg, beg));
+    items.clear();
+    beg.clear();
+    CKR(buildP2PItems(pl, kP2PMfmaTargets, items, beg));
     X.nitems = (int)items.size();
     X.nleaves = (int)pl.p2pLeaf.size();
     X.st.p2p_items = X.nitems;
     CKR(X.upv(X.items, items));
-    CKR(X.upv(X.itemBeg, itemBeg));
+    CKR(X.upv(X.itemBeg, beg));
   }
-  CKR(buildLaneItems(X, pl));
   {
     CKR(X.upv(X.leafCell, pl.p2pLeaf));
     CKR(X.upv(X.rb, pl.p2pSrcB));
@@ -2790,7 +2527,7 @@ static void launchP2PLane(Exec& X, hipStream_t s, int r0) {
   if (X.p2pPhase == kPhaseNone) go(std::integral_constant<int, kPhaseNone>());
   else if (X.p2pPhase == kPhaseTable) go(std::integral_constant<int, kPhaseTable>());
   else go(std::integral_constant<int, kPhaseLibrary>());
-  hipLaunchKernelGGL((k_p2p_lane_reduce<R, NR>), itemGrid(X.nleaves), dim3(64), 0, s,
+  hipLaunchKernelGGL((k_p2p_reduce<R, NR, kP2PTargets>), itemGrid(X.nleaves), dim3(64), 0, s,
                      X.laneItemBeg, X.leafCell, X.T.pbeg, X.T.nprt, (const double2*)X.partial, p,
                      (size_t)X.nt, X.nleaves);
 }
@@ -2799,16 +2536,18 @@ static void launchP2PLane(Exec& X, hipStream_t s, int r0) {
 static void launchP2PMfma(Exec& X, hipStream_t s, int r0) {
   const float2* q = (const float2*)X.q + (size_t)r0 * X.ns;
   float2* p = (float2*)X.p + (size_t)r0 * X.nt;
-  if (X.smallArg)
-    hipLaunchKernelGGL((k_p2p_mfma<true>), itemGrid(X.nitems), dim3(256), 0, s, X.items,
-                       X.leafCell, X.T.pbeg, X.T.nprt, X.tx, X.ty, X.tz, X.sx, X.sy, X.sz, q,
-                       (size_t)X.ns, X.rb, X.re, X.kappa, X.partial, X.nitems);
-  else
-    hipLaunchKernelGGL((k_p2p_mfma<false>), itemGrid(X.nitems), dim3(256), 0, s, X.items,
-                       X.leafCell, X.T.pbeg, X.T.nprt, X.tx, X.ty, X.tz, X.sx, X.sy, X.sz, q,
-                       (size_t)X.ns, X.rb, X.re, X.kappa, X.partial, X.nitems);
-  hipLaunchKernelGGL((k_p2p_reduce<float, kP2PMfmaNR>), itemGrid(X.nleaves), dim3(64), 0, s,
-                     X.itemBeg, X.items, X.leafCell, X.T.pbeg, X.T.nprt,
+  const P2PMfmaArgs A = {X.items, X.leafCell, X.T.pbeg, X.tx,  X.ty, X.tz, X.sx, X.sy, X.sz, q,
+                         (size_t)X.ns, X.rb, X.re, (const float2*)X.phaseTab, X.partial,
+                         X.nitems};
+  auto go = [&](auto phase) {
+    hipLaunchKernelGGL((k_p2p_mfma<decltype(phase)::value>),
+                       itemGrid(((int64_t)X.nitems + 3) / 4), dim3(256), 0, s, A, X.phaseConsts);
+  };
+  if (X.p2pPhase == kPhaseNone) go(std::integral_constant<int, kPhaseNone>());
+  else if (X.p2pPhase == kPhaseTable) go(std::integral_constant<int, kPhaseTable>());
+  else go(std::integral_constant<int, kPhaseLibrary>());
+  hipLaunchKernelGGL((k_p2p_reduce<float, kP2PMfmaNR, kP2PMfmaTargets>), itemGrid(X.nleaves),
+                     dim3(256), 0, s, X.itemBeg, X.leafCell, X.T.pbeg, X.T.nprt,
                      (const double2*)X.partial, p, (size_t)X.nt, X.nleaves);
 }
 

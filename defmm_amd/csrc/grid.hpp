@@ -6,8 +6,8 @@
 //  - Per-item kernels (one block per list item) use a 2D grid of at most
 //    kGridX blocks per row; a block's item index is y * gridDim.x + x, and the
 //    kernel returns for indices >= n.
-//  - Element-wise kernels (k_zero, k_zero_slots) loop with a grid stride over
-//    a grid capped at kZeroBlocks blocks.
+//  - Element-wise kernels (k_zero_slots, k_table_rows) loop with a grid stride
+//    over a grid capped at kZeroBlocks blocks.
 #pragma once
 #include <stdint.h>
 

@@ -1,4 +1,5 @@
-// Near field with a lane per source (1, 2, 3, 4 or 8 right-hand sides).
+// Near field: with a lane per source (1, 2, 3, 4 or 8 right-hand sides), and
+// on the matrix cores (16, float).
 //
 //   p_i += sum_j exp(i kappa r) / (4 pi r) q_j,  r = |x_i - y_j|,
 // term 0 when r^2 < 1e-16 (reference include/operators/P2P.hpp:42-79).
@@ -54,13 +55,20 @@ __device__ __forceinline__ void p2pValue(double x, double y, double z, const Pha
   }
 }
 
-// Work item of k_p2p_lane: nt <= kP2PTargets targets of one leaf, from t0
-// (leaf-relative), against cnt sources of its list from (range r, offset
-// off).
-constexpr int kP2PTargets = 8;
-struct P2PLaneItem {
+// Work item: nt targets of one leaf, from t0 (leaf-relative), against cnt
+// sources of its list from (range r, offset off).
+struct P2PItem {
   int leaf, t0, nt, r, off, cnt;
 };
+// Targets per item of k_p2p_lane, at most.
+constexpr int kP2PTargets = 8;
+// A leaf's n targets are cut into equal chunks of at most tg; tg itself where
+// an item works on whole row blocks of 16.
+DFM_HD inline int p2pChunk(int n, int tg) {
+  if (tg % 16 == 0) return tg;
+  const int chunks = (n + tg - 1) / tg;
+  return (n + chunks - 1) / chunks;
+}
 
 // Sum of v over the wave, N values (a power of two, at most 64) at once: each
 // halving step sends half of the values to the other half of the lanes, so N
@@ -118,7 +126,7 @@ constexpr int p2pSweep() {
 }
 template <typename R, int NR, int Phase>
 __global__ __launch_bounds__(256) void k_p2p_lane(
-    const P2PLaneItem* __restrict__ items, const int* __restrict__ leafCell,
+    const P2PItem* __restrict__ items, const int* __restrict__ leafCell,
     const int* __restrict__ tpbeg, const double* __restrict__ tx, const double* __restrict__ ty,
     const double* __restrict__ tz, const double* __restrict__ sx, const double* __restrict__ sy,
     const double* __restrict__ sz, const typename C2T<R>::T* __restrict__ q, size_t qStride,
@@ -140,7 +148,7 @@ __global__ __launch_bounds__(256) void k_p2p_lane(
   const int item = (int)(blockIdx.y * gridDim.x + blockIdx.x) * 4 +
                    __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   if (item >= nItems) return;
-  const P2PLaneItem it = items[item];
+  const P2PItem it = items[item];
   const int tb = tpbeg[leafCell[it.leaf]] + it.t0;
   for (int t0 = 0; t0 < it.nt; t0 += TC) {
     const int nt = min(TC, it.nt - t0);
@@ -245,11 +253,178 @@ __global__ __launch_bounds__(256) void k_p2p_lane(
   }
 }
 
+// 16 right-hand sides of the float path on the matrix cores.  An item's sums
+// are the product of the kernel matrix G (targets x sources, complex, one
+// element per lane and step, phase reduced in double) and the charges Q
+// (sources x 16):
+//   P_re += G_re Q_re - G_im Q_im,   P_im += G_re Q_im + G_im Q_re,
+// four V_MFMA_F32_16X16X4_F32 per 4 sources and 16 targets.  Operands: A (16
+// x 4) lane l holds row l % 16, column l / 16; B (4 x 16) row l / 16, column
+// l % 16; D (16 x 16) column l % 16, rows 4 (l / 16) + 0..3.  So lane l
+// evaluates G for target l % 16 of a row block and source 4 k + l / 16 of
+// step k, and ends with right-hand side l % 16 of targets 4 (l / 16) + 0..3.
+//
+// A wave per item of at most kP2PMfmaTargets targets (two row blocks, which
+// share the source operands), 4 items per block with the phase table in LDS.
+// The wave stages 16 sources at a time in LDS of its own: lane l loads source
+// l % 16 (coordinate l / 16, and right-hand sides l / 16 + 4 u), one step
+// ahead; no barrier, so no wave waits for another.  Every 64 sources the sums
+// are added to double ones.
+//
+// Bound by the SIMD's issue: 64 pairs take the matrix core 128 clocks and the
+// vector unit about 200 (34 instructions, 16 of them double), and on this chip
+// the two do not overlap, not even between waves (four waves of
+// V_MFMA_F32_16X16X4_F32 and 8 independent v_fma each: 74 clocks, 35 and 36
+// alone).  A block of 4 waves per 64 targets, with three barriers per 64
+// sources and polynomials of kappa r over [-pi/4, pi/4], took 5.2 ms where
+// this takes 4.0 (100,000-point ellipsoid at 64 wavelengths, Ncrit 97) and
+// 1.07 for 0.74 (20,000-point cube).
+constexpr int kP2PMfmaNR = 16, kP2PMfmaTargets = 32;
+struct P2PMfmaArgs {
+  const P2PItem* items;
+  const int *leafCell, *tpbeg;
+  const double *tx, *ty, *tz, *sx, *sy, *sz;
+  const float2* q;
+  size_t qStride;
+  const int *rb, *re;
+  const float2* phase;
+  double2* partial;
+  int nItems;
+};
+// One item with MB row blocks; lc and lq are the wave's stage, tab the
+// block's phase table.
+template <int Phase, int MB>
+__device__ __forceinline__ void p2pMfmaItem(const P2PMfmaArgs& A, const PhaseConsts& pc, int item,
+                                            const P2PItem& it, const float2* tab,
+                                            double (*lc)[16], float2 (*lq)[kP2PMfmaNR + 1]) {
+  typedef float v4f __attribute__((ext_vector_type(4)));
+  constexpr int kStage = 16;
+  const int lane = threadIdx.x & 63, lr = lane & 15, kq = lane >> 4;
+  const int tb = A.tpbeg[A.leafCell[it.leaf]] + it.t0;
+  // targets past the item's repeat its last; their sums are not written
+  double xt[MB], yt[MB], zt[MB];
+#pragma unroll
+  for (int b = 0; b < MB; b++) {
+    const int i = tb + min(16 * b + lr, it.nt - 1);
+    xt[b] = A.tx[i];
+    yt[b] = A.ty[i];
+    zt[b] = A.tz[i];
+  }
+  v4f dre[MB], dim[MB];
+  double ar[MB][4], ai[MB][4];
+#pragma unroll
+  for (int b = 0; b < MB; b++) {
+    dre[b] = dim[b] = v4f{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int v = 0; v < 4; v++) ar[b][v] = ai[b][v] = 0.;
+  }
+  // this lane's source (l % 16 of the stage): offset o of range [b0, b0 +
+  // len); past the item's end it keeps its last source (or the item's first),
+  // without charge
+  int rr = it.r, b0 = A.rb[rr], len = A.re[rr] - b0, o = it.off, j = b0 + o;
+  auto advance = [&](int pos, int by) {
+    if (pos >= it.cnt) return;
+    o += by;
+    while (o >= len) {
+      o -= len;
+      rr++;
+      b0 = A.rb[rr];
+      len = A.re[rr] - b0;
+    }
+    j = b0 + o;
+  };
+  const double* sc = kq == 0 ? A.sx : kq == 1 ? A.sy : A.sz;
+  const float2* ql = A.q + (size_t)kq * A.qStride;
+  double nc;
+  float2 nq[4];
+  auto load = [&]() {
+    nc = sc[j];
+#pragma unroll
+    for (int u = 0; u < 4; u++) nq[u] = ql[4 * u * A.qStride + j];
+  };
+  advance(lr, lr);
+  load();
+  for (int pos = 0; pos < it.cnt; pos += kStage) {
+    const bool valid = pos + lr < it.cnt;
+    // the wave's LDS accesses are ordered; the fences keep the compiler to it
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+    if (kq < 3) lc[kq][lr] = nc;
+#pragma unroll
+    for (int u = 0; u < 4; u++) lq[lr][kq + 4 * u] = valid ? nq[u] : make_float2(0.f, 0.f);
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+    advance(pos + kStage + lr, kStage);
+    load();
+#pragma unroll
+    for (int k = 0; k < kStage / 4; k++) {
+      const int s = 4 * k + kq;
+      const double xs = lc[0][s], ys = lc[1][s], zs = lc[2][s];
+      const float2 ch = lq[s][lr];
+      const float mi = -ch.y;
+#pragma unroll
+      for (int b = 0; b < MB; b++) {
+        float co, si;
+        p2pValue<Phase, float>(xt[b] - xs, yt[b] - ys, zt[b] - zs, pc, tab, co, si);
+        dre[b] = __builtin_amdgcn_mfma_f32_16x16x4f32(co, ch.x, dre[b], 0, 0, 0);
+        dim[b] = __builtin_amdgcn_mfma_f32_16x16x4f32(co, ch.y, dim[b], 0, 0, 0);
+        if constexpr (Phase != kPhaseNone) {
+          dre[b] = __builtin_amdgcn_mfma_f32_16x16x4f32(si, mi, dre[b], 0, 0, 0);
+          dim[b] = __builtin_amdgcn_mfma_f32_16x16x4f32(si, ch.x, dim[b], 0, 0, 0);
+        }
+      }
+    }
+    if ((pos & 48) == 48 || pos + kStage >= it.cnt) {
+#pragma unroll
+      for (int b = 0; b < MB; b++) {
+#pragma unroll
+        for (int v = 0; v < 4; v++) {
+          ar[b][v] += (double)dre[b][v];
+          ai[b][v] += (double)dim[b][v];
+        }
+        dre[b] = dim[b] = v4f{0.f, 0.f, 0.f, 0.f};
+      }
+    }
+  }
+  constexpr double kInv4Pi = 0.079577471545947667884;
+#pragma unroll
+  for (int b = 0; b < MB; b++)
+#pragma unroll
+    for (int v = 0; v < 4; v++) {
+      const int t = 16 * b + 4 * kq + v;
+      if (t < it.nt)
+        A.partial[((size_t)item * kP2PMfmaNR + lr) * kP2PMfmaTargets + t] =
+            make_double2(ar[b][v] * kInv4Pi, ai[b][v] * kInv4Pi);
+    }
+}
+// (at least 4 waves per SIMD: the sums then stay in registers that both kinds
+// of instruction take)
+template <int Phase>
+__global__ __launch_bounds__(256, 4) void k_p2p_mfma(P2PMfmaArgs A, PhaseConsts pc) {
+  __shared__ float2 tab[Phase == kPhaseTable ? kPhaseN : 1];
+  __shared__ double lc[4][3][16];
+  __shared__ float2 lq[4][16][kP2PMfmaNR + 1];
+  if constexpr (Phase == kPhaseTable) {
+    static_assert(kPhaseN == 256, "one table entry per thread");
+    tab[threadIdx.x] = A.phase[threadIdx.x];
+    __syncthreads();
+  }
+  const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int item = (int)(blockIdx.y * gridDim.x + blockIdx.x) * 4 + w;
+  if (item >= A.nItems) return;
+  const P2PItem it = A.items[item];
+  if (it.nt > 16) p2pMfmaItem<Phase, 2>(A, pc, item, it, tab, lc[w], lq[w]);
+  else p2pMfmaItem<Phase, 1>(A, pc, item, it, tab, lc[w], lq[w]);
+}
+
 // Adds the partial sums of a leaf's items to p: the leaf's targets are cut
-// into chunks of `chunk` (the last one smaller), its source list into runs;
-// item (run, chunk) of the leaf is itemBeg[leaf] + run * chunks + chunk.
-template <typename R, int NR>
-__global__ __launch_bounds__(64) void k_p2p_lane_reduce(
+// into chunks of p2pChunk(n, TG), its source list into runs; item (run,
+// chunk) of the leaf is itemBeg[leaf] + run * chunks + chunk, and its sum of
+// right-hand side r and target t is partial[(item * NR + r) * TG + t].
+template <typename R, int NR, int TG>
+__global__ void k_p2p_reduce(
     const int* __restrict__ itemBeg, const int* __restrict__ leafCell,
     const int* __restrict__ tpbeg, const int* __restrict__ tnprt,
     const double2* __restrict__ partial, typename C2T<R>::T* __restrict__ p, size_t pStride,
@@ -260,26 +435,20 @@ __global__ __launch_bounds__(64) void k_p2p_lane_reduce(
   const int c = leafCell[leaf];
   const int pb = tpbeg[c], n = tnprt[c];
   const int ib = itemBeg[leaf], ie = itemBeg[leaf + 1];
-  const int chunks = (n + kP2PTargets - 1) / kP2PTargets, chunk = (n + chunks - 1) / chunks;
-  for (int i = threadIdx.x; i < n; i += 64) {
+  const int chunks = (n + TG - 1) / TG, chunk = p2pChunk(n, TG);
+  for (int x = threadIdx.x; x < NR * n; x += blockDim.x) {
+    const int r = NR == 1 ? 0 : x / n, i = x - r * n;
     const int ch = i / chunk, t = i - ch * chunk;
-    double sr[NR], si[NR];
-#pragma unroll
-    for (int r = 0; r < NR; r++) sr[r] = si[r] = 0.;
-    for (int k = ib + ch; k < ie; k += chunks)
-#pragma unroll
-      for (int r = 0; r < NR; r++) {
-        const double2 v = partial[((size_t)k * NR + r) * kP2PTargets + t];
-        sr[r] += v.x;
-        si[r] += v.y;
-      }
-#pragma unroll
-    for (int r = 0; r < NR; r++) {
-      R2 o = p[r * pStride + pb + i];
-      o.x = (R)((double)o.x + sr[r]);
-      o.y = (R)((double)o.y + si[r]);
-      p[r * pStride + pb + i] = o;
+    double sr = 0., si = 0.;
+    for (int k = ib + ch; k < ie; k += chunks) {
+      const double2 v = partial[((size_t)k * NR + r) * TG + t];
+      sr += v.x;
+      si += v.y;
     }
+    R2 o = p[r * pStride + pb + i];
+    o.x = (R)((double)o.x + sr);
+    o.y = (R)((double)o.y + si);
+    p[r * pStride + pb + i] = o;
   }
 }
 

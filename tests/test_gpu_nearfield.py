@@ -70,3 +70,29 @@ def test_right_hand_side_counts_match_single(nr):
         l2, mx = _diff(P, single)
         _say(f"  precision {prec}: batch vs single rel L2 {l2:.3e} max {mx:.3e}")
         assert l2 <= tol and mx <= 10 * tol
+
+
+# 16 right-hand sides take the matrix cores (float): row blocks of 16 targets,
+# two per item, stages of 16 sources, sums to double every 64.  Single
+# evaluations (compared with the oracle above) round the same float values in
+# another order: the bounds of the test above.
+@pytest.mark.parametrize("kappa", [0.0, 6.0, 1e-31])
+@pytest.mark.parametrize("n,ncrit", [(900, 4), (1500, 18), (2500, 34), (3000, 130)])
+def test_sixteen_right_hand_sides(n, ncrit, kappa):
+    import defmm_amd as dm
+    from defmm_amd import workloads as wl
+    src = wl.sphere(n, seed=23)
+    trg = np.concatenate([wl.sphere(n // 2 + 3, seed=6), src[:40]])  # some targets are sources
+    nr = 17
+    Q = np.stack([wl.charges(n, seed=60 + r) for r in range(nr)])
+    _say(f"case: sphere N={n} Ncrit={ncrit} kappa={kappa}, {nr} right-hand sides")
+    A = _plan(dm, src, trg, 3, ncrit, kappa, dm.MIXED)
+    single = np.stack([A.apply(Q[r]) for r in range(nr)])
+    A.set_rhs(nr)
+    P = A.apply_batch(Q)
+    again = A.apply_batch(Q)
+    A.destroy()
+    l2, mx = _diff(P, single)
+    _say(f"  batch vs single rel L2 {l2:.3e} max {mx:.3e}")
+    assert l2 <= 1e-6 and mx <= 1e-5
+    assert np.array_equal(P, again)
