@@ -699,20 +699,35 @@ __global__ __launch_bounds__(256) void k_m2f(const int* __restrict__ m2fSlot,
 // in h to the axis-order index s (permutations.hpp:87-120).
 static const int kVariantOfSigma[8] = {0, 1, 0, 2, 3, 0, 4, 5};
 
-// Workgroups are dealt to the 8 XCDs in turn.  Each XCD gets a contiguous part
-// of the (level, direction, cell) group order, so that its L2 sees the groups
-// that share source rows; the parts hold equal shares of the rows to load
-// (m2lParts), not of the groups: equal counts gave the XCDs with the dense
-// levels up to 1.7 times the mean (20,000-point cube at 32 wavelengths), and
-// the others idled.  Block b takes item at[b mod 8] + b / 8, if it is in the
-// part (-1 otherwise).
+// Workgroups are dealt to the 8 XCDs in turn.  The (level, direction, cell)
+// group order is cut into segments, each into 8 contiguous parts, one per XCD:
+// an XCD's L2 sees the groups that share source rows, and all XCDs read the
+// same segment's table rows at a time.  Segments and parts hold equal shares
+// of the rows to load (m2lParts), not of the groups.  Block b belongs to XCD
+// b mod 8 and takes item b / 8 of that XCD's parts, counted over the segments
+// (-1 past the last).
+//
+// Rows alone do not predict the time (a level's rows may or may not be in the
+// caches): with one segment the XCDs ended at 1.00 to 1.39 ms of 1.47
+// (100,000-point ellipsoid, order 6), at 1.95 to 2.40 (20,000-point cube,
+// order 8) and at 16.6 to 19.3 (1,000,000-point sphere, order 7).  With 8 they
+// end within 5% of one another: 1.43 -> 1.31, 2.39 -> 2.20 and 18.9 -> 17.6 ms
+// (4: 2.26 and 17.8; 16: 2.29 and 17.9).
+constexpr int kXcdSegments = 8;    // at most
+constexpr int kXcdPartGroups = 128;  // groups of a part, at least (on average)
 struct XcdParts {
-  int at[9];
+  int segments;
+  int at[8 * kXcdSegments + 1];  // first group of part 8 * segment + XCD
 };
 __device__ __forceinline__ int partItem(const XcdParts& p, int b) {
   const int x = b & 7;
-  const int i = p.at[x] + (b >> 3);
-  return i < p.at[x + 1] ? i : -1;
+  int i = b >> 3;
+  for (int s = 0; s < p.segments; s++) {
+    const int a = p.at[8 * s + x], n = p.at[8 * s + x + 1] - a;
+    if (i < n) return a + i;
+    i -= n;
+  }
+  return -1;
 }
 
 // M2L block shape for order L: NW frequencies per thread (at most 3 where a
@@ -2449,24 +2464,27 @@ static int upload(Exec& X, Plan& pl) {
 
 static inline unsigned nblk(int64_t n, int b) { return (unsigned)((n + b - 1) / b); }
 
-// Launchers of the NR-wide kernels: the widest NR in {8, 4, 2, 1} that is
-// <= n and allowed, for right-hand sides r0 .. r0 + NR - 1.
-// Groups g0 .. g0 + ng - 1 (counted from g0) in 8 contiguous parts of equal
-// cost; grid: 8 times the largest part.
+// The parts of groups g0 .. g0 + ng - 1 (counted from g0); grid: 8 times the
+// blocks of the XCD with the most groups.
 static XcdParts m2lParts(const Exec& X, int g0, int ng, int64_t& grid) {
   XcdParts p;
+  p.segments = std::max(1, std::min(kXcdSegments, ng / (8 * kXcdPartGroups)));
+  const int n = 8 * p.segments;
   const auto first = X.hGroupCost.begin() + g0;
   const int64_t c0 = *first, total = first[ng] - c0;
   p.at[0] = 0;
-  p.at[8] = ng;
-  for (int x = 1; x < 8; x++)
-    p.at[x] = (int)(std::lower_bound(first, first + ng, c0 + total * x / 8) - first);
-  grid = 0;
-  for (int x = 0; x < 8; x++) grid = std::max<int64_t>(grid, p.at[x + 1] - p.at[x]);
-  grid *= 8;
+  p.at[n] = ng;
+  for (int x = 1; x < n; x++)
+    p.at[x] = (int)(std::lower_bound(first, first + ng, c0 + total / n * x + total % n * x / n) -
+                    first);
+  int64_t blocks[8] = {};
+  for (int x = 0; x < n; x++) blocks[x & 7] += p.at[x + 1] - p.at[x];
+  grid = 8 * *std::max_element(blocks, blocks + 8);
   return p;
 }
 
+// Launchers of the NR-wide kernels: the widest NR in {8, 4, 2, 1} that is
+// <= n and allowed, for right-hand sides r0 .. r0 + NR - 1.
 template <typename R, int L, int NR>
 static void launchM2L(Exec& X, hipStream_t s, int g0, int ng, const typename C2T<R>::T* F,
                       typename C2T<R>::T* Lb, const OpConsts<R>& oc) {
