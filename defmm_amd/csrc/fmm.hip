@@ -713,15 +713,28 @@ static const int kVariantOfSigma[8] = {0, 1, 0, 2, 3, 0, 4, 5};
 // order 8) and at 16.6 to 19.3 (1,000,000-point sphere, order 7).  With 8 they
 // end within 5% of one another: 1.43 -> 1.31, 2.39 -> 2.20 and 18.9 -> 17.6 ms
 // (4: 2.26 and 17.8; 16: 2.29 and 17.9).
-constexpr int kXcdSegments = 8;    // at most
+//
+// A launch covers up to kXcdChunks chunks of right-hand sides, chunk after
+// chunk; XCD x takes parts (x + chunk) mod 8, so that what still differs
+// between the parts evens out, and one chunk's tail overlaps the next's start:
+// 16 right-hand sides, ellipsoid 10.5 -> 9.8 ms, cube at order 4 1.28 -> 1.17,
+// at order 8 15.9 -> 15.5 (a launch per chunk before).
+constexpr int kXcdSegments = 8;      // at most
 constexpr int kXcdPartGroups = 128;  // groups of a part, at least (on average)
+constexpr int kXcdChunks = 8;
 struct XcdParts {
-  int segments;
-  int at[8 * kXcdSegments + 1];  // first group of part 8 * segment + XCD
+  int segments, chunks;
+  int total[8];                  // groups of part x, all segments
+  int at[8 * kXcdSegments + 1];  // first group of part x in segment s: at[8 s + x]
 };
-__device__ __forceinline__ int partItem(const XcdParts& p, int b) {
-  const int x = b & 7;
-  int i = b >> 3;
+__device__ __forceinline__ int partItem(const XcdParts& p, int b, int& chunk) {
+  int x = b & 7, i = b >> 3;
+  chunk = 0;
+  while (i >= p.total[x]) {
+    i -= p.total[x];
+    x = (x + 1) & 7;
+    if (++chunk >= p.chunks) return -1;
+  }
   for (int s = 0; s < p.segments; s++) {
     const int a = p.at[8 * s + x], n = p.at[8 * s + x + 1] - a;
     if (i < n) return a + i;
@@ -880,8 +893,11 @@ __global__ __launch_bounds__((M2LShapeN<R, L, NR>::TB)) void k_m2l(
   constexpr int NU = G * NR, NB = f2lBatch(NU);
   __shared__ R2 J[NB * PP], T1[NB * L * P * P];
   const int tid = threadIdx.x;
-  const int grp = partItem(parts, itemIndex());
+  int chunk;
+  const int grp = partItem(parts, itemIndex(), chunk);
   if (grp < 0) return;
+  F += (size_t)chunk * NR * fStride;
+  Lout += (size_t)chunk * NR * lStride;
   // units of this thread, clamped to the row: every load is in bounds and
   // unconditional, and the accumulators of w >= PP are never stored
   unsigned wl[NW];
@@ -1027,8 +1043,11 @@ __global__ __launch_bounds__(M2LShape<L>::TB) void k_m2l_col(
   constexpr int NT = P == 15 ? NR : 1;
   __shared__ R2 T1[NT][L * P2], T2[NT][L * L * P];
   const int tid = threadIdx.x;
-  const int grp = partItem(parts, itemIndex());
+  int chunk;
+  const int grp = partItem(parts, itemIndex(), chunk);
   if (grp < 0) return;
+  F += (size_t)chunk * NR * fStride;
+  Lout += (size_t)chunk * NR * lStride;
   // threads beyond the cube's columns load a valid column and store nothing
   const int col = min(tid, P2 - 1);
   R2 acc[P][NR];
@@ -1123,7 +1142,8 @@ __global__ __launch_bounds__(M2LShape<L>::TB) void k_m2l_fly(const int* __restri
   __shared__ R2 sM[LL], B1[NB], B2[NB], J[PP];
   __shared__ R wc[P], ws[P];
   const int tid = threadIdx.x;
-  const int grp = partItem(parts, itemIndex());
+  int chunk;  // (one)
+  const int grp = partItem(parts, itemIndex(), chunk);
   if (grp < 0) return;
   if (tid < P) {
     wc[tid] = twc[tid];
@@ -2464,11 +2484,12 @@ static int upload(Exec& X, Plan& pl) {
 
 static inline unsigned nblk(int64_t n, int b) { return (unsigned)((n + b - 1) / b); }
 
-// The parts of groups g0 .. g0 + ng - 1 (counted from g0); grid: 8 times the
-// blocks of the XCD with the most groups.
-static XcdParts m2lParts(const Exec& X, int g0, int ng, int64_t& grid) {
-  XcdParts p;
+// The parts of groups g0 .. g0 + ng - 1 (counted from g0) for `chunks` chunks
+// of right-hand sides; grid: 8 times the blocks of the XCD with the most.
+static XcdParts m2lParts(const Exec& X, int g0, int ng, int chunks, int64_t& grid) {
+  XcdParts p{};
   p.segments = std::max(1, std::min(kXcdSegments, ng / (8 * kXcdPartGroups)));
+  p.chunks = chunks;
   const int n = 8 * p.segments;
   const auto first = X.hGroupCost.begin() + g0;
   const int64_t c0 = *first, total = first[ng] - c0;
@@ -2477,56 +2498,61 @@ static XcdParts m2lParts(const Exec& X, int g0, int ng, int64_t& grid) {
   for (int x = 1; x < n; x++)
     p.at[x] = (int)(std::lower_bound(first, first + ng, c0 + total / n * x + total % n * x / n) -
                     first);
-  int64_t blocks[8] = {};
-  for (int x = 0; x < n; x++) blocks[x & 7] += p.at[x + 1] - p.at[x];
-  grid = 8 * *std::max_element(blocks, blocks + 8);
+  for (int x = 0; x < n; x++) p.total[x & 7] += p.at[x + 1] - p.at[x];
+  grid = 0;
+  for (int x = 0; x < 8; x++) {
+    int64_t blocks = 0;
+    for (int c = 0; c < chunks; c++) blocks += p.total[(x + c) & 7];
+    grid = std::max(grid, 8 * blocks);
+  }
   return p;
 }
 
-// Launchers of the NR-wide kernels: the widest NR in {8, 4, 2, 1} that is
-// <= n and allowed, for right-hand sides r0 .. r0 + NR - 1.
+// M2L of groups g0 .. g0 + ng - 1 for `chunks` chunks of NR right-hand sides.
 template <typename R, int L, int NR>
-static void launchM2L(Exec& X, hipStream_t s, int g0, int ng, const typename C2T<R>::T* F,
-                      typename C2T<R>::T* Lb, const OpConsts<R>& oc) {
+static void launchM2L(Exec& X, hipStream_t s, int g0, int ng, int chunks,
+                      const typename C2T<R>::T* F, typename C2T<R>::T* Lb, const OpConsts<R>& oc) {
   typedef typename C2T<R>::T R2;
   constexpr int G = M2LShapeN<R, L, NR>::G;
   int64_t grid = 0;
-  const XcdParts parts = m2lParts(X, g0, ng, grid);
-  if constexpr (M2LShape<L>::kColumns)
-    hipLaunchKernelGGL((k_m2l_col<R, L, NR>), itemGrid(grid), dim3(M2LShape<L>::TB), 0, s,
-                       X.gBeg + g0, X.gTarget + (size_t)g0 * G, X.gSrc, X.gMask, X.gCode, F,
-                       X.fStride, (const R2*)X.U, Lb, X.lStride, oc.twc, oc.tws, parts);
-  else if (X.m2lSliced)
-    hipLaunchKernelGGL((k_m2l<R, L, NR, true>), itemGrid(grid), dim3(M2LShapeN<R, L, NR>::TB), 0, s,
-                       X.gBeg + g0, X.gTarget + (size_t)g0 * G, X.gSrc, X.gMask, X.gCode, F,
-                       X.fStride, (const R2*)X.U, Lb, X.lStride, oc.twc, oc.tws, parts);
-  else
-    hipLaunchKernelGGL((k_m2l<R, L, NR, false>), itemGrid(grid), dim3(M2LShapeN<R, L, NR>::TB), 0, s,
-                       X.gBeg + g0, X.gTarget + (size_t)g0 * G, X.gSrc, X.gMask, X.gCode, F,
-                       X.fStride, (const R2*)X.U, Lb, X.lStride, oc.twc, oc.tws, parts);
+  const XcdParts parts = m2lParts(X, g0, ng, chunks, grid);
+  auto go = [&](auto kernel, int tb) {
+    hipLaunchKernelGGL(kernel, itemGrid(grid), dim3(tb), 0, s, X.gBeg + g0,
+                       X.gTarget + (size_t)g0 * G, X.gSrc, X.gMask, X.gCode, F, X.fStride,
+                       (const R2*)X.U, Lb, X.lStride, oc.twc, oc.tws, parts);
+  };
+  if constexpr (M2LShape<L>::kColumns) go(k_m2l_col<R, L, NR>, M2LShape<L>::TB);
+  else if (X.m2lSliced) go(k_m2l<R, L, NR, true>, M2LShapeN<R, L, NR>::TB);
+  else go(k_m2l<R, L, NR, false>, M2LShapeN<R, L, NR>::TB);
 }
 
-// Right-hand sides of the next M2L launch when n are left.
+// Right-hand sides per F row read (the NR of the next M2L launch) when n are
+// left: the widest of {8, 4, 2, 1} that is <= n and allowed.
 template <typename R, int L>
 constexpr int m2lChunkWidth(int n) {
   constexpr int mx = m2lMaxNR<R, L>();
   return (mx >= 8 && n >= 8) ? 8 : (mx >= 4 && n >= 4) ? 4 : (mx >= 2 && n >= 2) ? 2 : 1;
 }
 
-// M2L of groups g0 .. g0 + ng - 1 for right-hand sides r0 .. r0 + n' - 1
-// (n' = m2lChunkWidth(n), returned); their F rows start at F (right-hand
-// side r0 + i at F + i * fStride).
+// M2L of groups g0 .. g0 + ng - 1 for the right-hand sides of one launch, from
+// r0 on; returns their number: m2lChunkWidth(n) times at most `chunks` chunks
+// of that width.  Their F rows start at F (right-hand side r0 + i at F + i *
+// fStride).
 template <typename R, int L>
-static int m2lChunk(Exec& X, hipStream_t s, int g0, int ng, int r0, int n, const OpConsts<R>& oc,
-                    const typename C2T<R>::T* F) {
+static int m2lLaunch(Exec& X, hipStream_t s, int g0, int ng, int r0, int n, int chunks,
+                     const OpConsts<R>& oc, const typename C2T<R>::T* F) {
   typedef typename C2T<R>::T R2;
   R2* Lb = (R2*)X.Lb + (size_t)r0 * X.lStride;
   constexpr int mx = m2lMaxNR<R, L>();
-  if (mx >= 8 && n >= 8) { launchM2L<R, L, (mx >= 8 ? 8 : 1)>(X, s, g0, ng, F, Lb, oc); return 8; }
-  if (mx >= 4 && n >= 4) { launchM2L<R, L, (mx >= 4 ? 4 : 1)>(X, s, g0, ng, F, Lb, oc); return 4; }
-  if (mx >= 2 && n >= 2) { launchM2L<R, L, (mx >= 2 ? 2 : 1)>(X, s, g0, ng, F, Lb, oc); return 2; }
-  launchM2L<R, L, 1>(X, s, g0, ng, F, Lb, oc);
-  return 1;
+  const int w = m2lChunkWidth<R, L>(n);
+  // (the block index of all chunks together stays an int)
+  const int c = (int)std::min<int64_t>({(int64_t)chunks, (int64_t)n / w, (int64_t)kXcdChunks,
+                                        std::max<int64_t>(1, INT32_MAX / 16 / std::max(1, ng))});
+  if (w == 8) launchM2L<R, L, (mx >= 8 ? 8 : 1)>(X, s, g0, ng, c, F, Lb, oc);
+  else if (w == 4) launchM2L<R, L, (mx >= 4 ? 4 : 1)>(X, s, g0, ng, c, F, Lb, oc);
+  else if (w == 2) launchM2L<R, L, (mx >= 2 ? 2 : 1)>(X, s, g0, ng, c, F, Lb, oc);
+  else launchM2L<R, L, 1>(X, s, g0, ng, c, F, Lb, oc);
+  return w * c;
 }
 
 // NR right-hand sides with a lane per source
@@ -2670,11 +2696,11 @@ static int runTyped(Exec& X, const double2* qin, double2* pout, int parts, int n
     if (stored) {
       // L (aliasing M) is written for every target slot from here on
       for (int r0 = 0; r0 < nrhs;)
-        r0 += m2lChunk<R, L>(X, s, 0, X.nGroups, r0, nrhs - r0, oc, Fr(r0));
+        r0 += m2lLaunch<R, L>(X, s, 0, X.nGroups, r0, nrhs - r0, kXcdChunks, oc, Fr(r0));
     } else if (X.m2lMode == DEFMM_M2L_ON_THE_FLY) {
       if constexpr (!M2LShape<L>::kColumns) {
         int64_t grid = 0;
-        const XcdParts all = m2lParts(X, 0, X.nGroups, grid);
+        const XcdParts all = m2lParts(X, 0, X.nGroups, 1, grid);
         for (int r = 0; r < nrhs; r++)
           hipLaunchKernelGGL((k_m2l_fly<R, L>), itemGrid(grid), dim3(M2LShape<L>::TB), 0, s,
                              X.gBeg, X.gTarget, X.gSrc, X.gMask, X.gCode, (const R2*)Mr(r),
@@ -2697,7 +2723,7 @@ static int runTyped(Exec& X, const double2* qin, double2* pout, int parts, int n
         for (int r0 = 0; r0 < nrhs;) {
           const int c = m2lChunkWidth<R, L>(nrhs - r0);
           launchM2F(X.bRows + w0, w1 - w0, r0, c, Fr(0));
-          r0 += m2lChunk<R, L>(X, s, g0, g1 - g0, r0, c, oc, Fr(0));
+          r0 += m2lLaunch<R, L>(X, s, g0, g1 - g0, r0, c, 1, oc, Fr(0));
         }
       }
     }
