@@ -199,9 +199,13 @@ __global__ __launch_bounds__(128) void k_p2m(const int2* __restrict__ items, Dev
 // wave w takes the range's slots w mod 4.  For a slot the wave writes W (64
 // points x 16 right-hand sides) to LDS, then for every 16-row block of L^3
 // runs ceil(n / 4) steps of V_MFMA_F32_16X16X4_F32 for the real and the
-// imaginary part (A: lane l row I = 16 m + l % 16, point 4 k + l / 16, the
-// product of the point's three 1D weights; B: point 4 k + l / 16,
-// right-hand side l % 16) and stores the 16 x 16 result times conj(sig2_s).
+// imaginary part (A: right-hand side l % 16, point 4 k + l / 16; B: lane l
+// point 4 k + l / 16, column I = 16 m + l % 16, the product of the point's
+// three 1D weights) and stores the 16 x 16 result times conj(sig2_s): lane l
+// holds I = 16 m + l % 16 of right-hand sides 4 (l / 16) + 0..3, so a store
+// covers whole 128-byte lines (with the operands the other way round, 8 bytes
+// of every 32; that and four steps a time instead of one: 100,000-point
+// ellipsoid, order 6, 2.36 -> 1.95 ms, 20,000-point cube, order 8, 2.37 -> 1.66).
 constexpr int kP2MMfmaNR = 16, kP2MMfmaSlots = 32, kP2MMfmaPoints = 64;
 template <int L>
 __global__ __launch_bounds__(256) void k_p2m_mfma(
@@ -283,21 +287,24 @@ __global__ __launch_bounds__(256) void k_p2m_mfma(
       const int a0 = rowOn ? I / (L * L) : 0, a1 = rowOn ? (I / L) % L : 0,
                 a2 = rowOn ? I % L : 0;
       mfma_v4f dre = {0.f, 0.f, 0.f, 0.f}, dim = {0.f, 0.f, 0.f, 0.f};
-      for (int ks = 0; ks < ksn; ks++) {
-        const int k = 4 * ks + j;
-        const float a = rowOn ? Wt[0][k][a0] * Wt[1][k][a1] * Wt[2][k][a2] : 0.f;
-        const float2 b = Bw[wave][k][lr];
-        dre = __builtin_amdgcn_mfma_f32_16x16x4f32(a, b.x, dre, 0, 0, 0);
-        dim = __builtin_amdgcn_mfma_f32_16x16x4f32(a, b.y, dim, 0, 0, 0);
-      }
-      // rows 16 mt + 4 j + v, right-hand side lr
+      // (four steps' LDS reads together; points past n have weight 0)
+      for (int ks = 0; ks < ksn; ks += 4)
 #pragma unroll
-      for (int v = 0; v < 4; v++) {
-        const int Io = 16 * mt + 4 * j + v;
-        if (Io < LL) {
+        for (int v = 0; v < 4; v++) {
+          const int k = 4 * (ks + v) + j;
+          const float a = Wt[0][k][a0] * Wt[1][k][a1] * Wt[2][k][a2];
+          const float2 b = Bw[wave][k][lr];
+          dre = __builtin_amdgcn_mfma_f32_16x16x4f32(b.x, a, dre, 0, 0, 0);
+          dim = __builtin_amdgcn_mfma_f32_16x16x4f32(b.y, a, dim, 0, 0, 0);
+        }
+      // weight index I, right-hand sides 4 j + v
+      if (rowOn) {
+        const float2 sg = hf ? sgr[I] : make_float2(1.f, 0.f);
+#pragma unroll
+        for (int v = 0; v < 4; v++) {
           float2 val = make_float2(dre[v], dim[v]);
-          if (hf) val = cmulc(val, sgr[Io]);
-          M[(size_t)lr * mStride + (size_t)sl * LL + Io] = val;
+          if (hf) val = cmulc(val, sg);
+          M[(size_t)(4 * j + v) * mStride + (size_t)sl * LL + I] = val;
         }
       }
     }
@@ -1439,11 +1446,14 @@ __global__ __launch_bounds__(256) void k_l2p(const int* __restrict__ leaves, Dev
 // L_s,r[I]; then p_r[i] += exp(i kappa d_s.(x_i - c)) C_s[i][r] (the sums of
 // L2P.hpp:121-173).  One block of 4 waves per (leaf, tile of up to TP
 // points): the tile's S is staged in LDS once for all slots; wave w takes
-// the slots k = w mod 4, each as ceil(L^3 / 4) steps of V_MFMA_F32_16X16X4_F32
-// (real and imaginary part of B, TP / 16 row blocks sharing each B operand)
-// with A = S (lane l: point l % 16 of a row block, weight index 4 k + l / 16)
-// and B (lane l: weight index 4 k + l / 16, right-hand side l % 16).  The
-// waves' sums are added in wave order at the end (deterministic).
+// the slots k = w mod 4, each as 4 ceil(L^3 / 16) steps of
+// V_MFMA_F32_16X16X4_F32 (real and imaginary part of B, TP / 16 row blocks
+// sharing each B operand) with A = S (lane l: point l % 16 of a row block) and
+// B (lane l: right-hand side l % 16).  The waves' sums are added in wave order
+// at the end (deterministic).  With rows of S 4 ceil(L^3 / 4) floats apart (512
+// at order 8: all rows on one bank) and 8-byte loads it took 1.10 ms where it
+// takes 0.82 (100,000-point ellipsoid, order 6) and 2.47 for 1.80 (20,000-point
+// cube, order 8).
 constexpr int kL2PMfmaNR = 16;
 template <int L>
 constexpr int l2pMfmaTile() {
@@ -1456,12 +1466,13 @@ __global__ __launch_bounds__(256) void k_l2p_mfma(
     const double* __restrict__ dirs, const float2* __restrict__ sig2,
     const float2* __restrict__ Lst, size_t lStride, OpConsts<float> oc, double kappa,
     float2* __restrict__ p, size_t pStride, int nItems) {
-  constexpr int LL = L * L * L, KS = (LL + 3) / 4, TP = l2pMfmaTile<L>(), NB = TP / 16;
-  // S (TP x 4 KS floats) and, once every wave is past the slot loop, the
-  // waves' sums (4 x TP x 16 complex) share one array
-  constexpr int NS = TP * KS * 4, NRED = 4 * TP * kL2PMfmaNR * 2;
-  __shared__ float smem[NS > NRED ? NS : NRED];
-  float(*S)[KS * 4] = reinterpret_cast<float(*)[KS * 4]>(smem);
+  constexpr int LL = L * L * L, KG = (LL + 15) / 16, TP = l2pMfmaTile<L>(), NB = TP / 16;
+  // S (TP rows of 16 KG floats, 4 more to spread 16 rows over the banks) and,
+  // once every wave is past the slot loop, the waves' sums (4 x TP x 16
+  // complex) share one array
+  constexpr int SW = 16 * KG + 4, NS = TP * SW, NRED = 4 * TP * kL2PMfmaNR * 2;
+  __shared__ __align__(16) float smem[NS > NRED ? NS : NRED];
+  float(*S)[SW] = reinterpret_cast<float(*)[SW]>(smem);
   float2(*red)[TP][kL2PMfmaNR] = reinterpret_cast<float2(*)[TP][kL2PMfmaNR]>(smem);
   __shared__ float W[3][TP][L];
   __shared__ double rel[3][TP];
@@ -1500,8 +1511,8 @@ __global__ __launch_bounds__(256) void k_l2p_mfma(
     for (int a = 0; a < L; a++) W[2][i][a] = t[a];
   }
   __syncthreads();
-  for (int x = tid; x < TP * KS * 4; x += 256) {
-    const int i = x / (KS * 4), I = x - i * (KS * 4);
+  for (int x = tid; x < TP * KG * 16; x += 256) {
+    const int i = x / (KG * 16), I = x - i * (KG * 16);
     float v = 0.f;
     if (I < LL) v = W[0][i][I / (L * L)] * W[1][i][(I / L) % L] * W[2][i][I % L];
     S[i][I] = v;
@@ -1524,30 +1535,58 @@ __global__ __launch_bounds__(256) void k_l2p_mfma(
       cre[b] = mfma_v4f{0.f, 0.f, 0.f, 0.f};
       cim[b] = mfma_v4f{0.f, 0.f, 0.f, 0.f};
     }
-    // KU steps' loads of L and of the phase row are issued together, ahead
-    // of their matrix-core steps (one load in flight per step would leave
-    // the loop bound by the load latency)
-    constexpr int KU = 8;
-    for (int ks0 = 0; ks0 < KS; ks0 += KU) {
-      float2 lv2[KU], sv[KU];
+    // 16 weight indices a group: lane l takes 16 g + 4 (l / 16) + 0..3, so
+    // that L, the phase row and S are read 16 bytes at a time (any assignment
+    // of indices to steps does, the same for A and B).  KU groups' loads are
+    // issued together, ahead of their matrix-core steps (with one in flight
+    // the load latency would bound the loop).
+    constexpr int KU = 2;
+    struct alignas(8) Two {
+      float2 v[2];
+    };
+    for (int g0 = 0; g0 < KG; g0 += KU) {
+      float2 lv2[KU][4], sv[KU][4];
 #pragma unroll
       for (int u = 0; u < KU; u++) {
-        const int kk = 4 * (ks0 + u) + j;
-        const bool on = ks0 + u < KS && kk < LL;
-        lv2[u] = on ? Ls[kk] : make_float2(0.f, 0.f);
-        sv[u] = (on && hf) ? sg[kk] : make_float2(1.f, 0.f);
+        const int kk = 16 * (g0 + u) + 4 * j;
+        if (kk + 4 <= LL) {
+#pragma unroll
+          for (int h = 0; h < 2; h++) {
+            const Two l = *(const Two*)(Ls + kk + 2 * h);
+            lv2[u][2 * h] = l.v[0];
+            lv2[u][2 * h + 1] = l.v[1];
+            if (hf) {
+              const Two p2 = *(const Two*)(sg + kk + 2 * h);
+              sv[u][2 * h] = p2.v[0];
+              sv[u][2 * h + 1] = p2.v[1];
+            }
+          }
+        } else {
+#pragma unroll
+          for (int e = 0; e < 4; e++) {
+            const bool on = kk + e < LL;
+            lv2[u][e] = on ? Ls[kk + e] : make_float2(0.f, 0.f);
+            if (hf) sv[u][e] = on ? sg[kk + e] : make_float2(1.f, 0.f);
+          }
+        }
       }
       __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
       for (int u = 0; u < KU; u++) {
-        if (ks0 + u >= KS) break;
-        const int kk = 4 * (ks0 + u) + j;
-        const float2 bv = hf ? cmul(lv2[u], sv[u]) : lv2[u];
+        if (g0 + u >= KG) break;
+        float4 a[NB];
 #pragma unroll
-        for (int b = 0; b < NB; b++) {
-          const float a = S[16 * b + lr][kk];
-          cre[b] = __builtin_amdgcn_mfma_f32_16x16x4f32(a, bv.x, cre[b], 0, 0, 0);
-          cim[b] = __builtin_amdgcn_mfma_f32_16x16x4f32(a, bv.y, cim[b], 0, 0, 0);
+        for (int b = 0; b < NB; b++)
+          a[b] = *(const float4*)&S[16 * b + lr][16 * (g0 + u) + 4 * j];
+#pragma unroll
+        for (int e = 0; e < 4; e++) {
+          const float2 bv = hf ? cmul(lv2[u][e], sv[u][e]) : lv2[u][e];
+#pragma unroll
+          for (int b = 0; b < NB; b++) {
+            const float w = e == 0 ? a[b].x : e == 1 ? a[b].y : e == 2 ? a[b].z : a[b].w;
+            cre[b] = __builtin_amdgcn_mfma_f32_16x16x4f32(w, bv.x, cre[b], 0, 0, 0);
+            cim[b] = __builtin_amdgcn_mfma_f32_16x16x4f32(w, bv.y, cim[b], 0, 0, 0);
+          }
         }
       }
     }
@@ -2608,8 +2647,10 @@ static void launchP2PMfma(Exec& X, hipStream_t s, int r0) {
 
 // One evaluation pass for nrhs <= X.nr right-hand sides: qin / pout hold
 // nrhs x n complex128 values, right-hand side after right-hand side, in
-// input order.  Stages as in the reference's gemv; M2L and P2P process up to
-// 8 right-hand sides per launch, the other stages one per launch.
+// input order.  Stages as in the reference's gemv.  P2M, L2P and P2P go by
+// groups of right-hand sides (16 on the matrix cores in float; P2P up to 8
+// per kernel value otherwise, P2M and L2P one), M2L by m2lLaunch, the other
+// stages take all in one launch.
 template <typename R, int L>
 static int runTyped(Exec& X, const double2* qin, double2* pout, int parts, int nrhs,
                     hipStream_t s) {

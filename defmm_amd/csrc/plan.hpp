@@ -44,14 +44,12 @@ struct NoInitAlloc : std::allocator<T> {
 typedef std::vector<int, NoInitAlloc<int>> ListVec;
 
 // Target slots per M2L work group: a thread holds one accumulator per group
-// target and frequency it owns (2 targets at L = 8, where a thread owns 4
-// frequencies, so that the FP64 kernel fits its registers; 3 at L = 7, where
-// the float kernel with two right-hand sides then fits two 768-thread blocks
-// per CU: 1M points / 16 wavelengths, 4 right-hand sides 182.8 -> 159.8 ms,
-// FP64 89.1 -> 91.4 ms; 1 from L = 8, where a thread owns a whole column of
-// 2L - 1 frequencies: at 20,000 points / 32 wavelengths / L = 8 the column
-// kernel took M2L from 3.41 to 2.44 ms in float (16 right-hand sides: 38.8 ->
-// 34.8 ms) and from 4.93 to 5.15 ms in double, against groups of 2).
+// target and frequency it owns.  3 at L = 7, where four would leave the float
+// kernel with two right-hand sides half the waves (1M points / 16 wavelengths,
+// 4 right-hand sides, 182.8 -> 159.8 ms; FP64 89.1 -> 91.4 ms); 1 from L = 8,
+// where a thread owns a whole column of 2L - 1 frequencies (20,000 points / 32
+// wavelengths / L = 8, float, 16 right-hand sides: M2L 17.0 ms where the
+// grouped kernel takes 18.3; one right-hand side 1.42 and 1.34).
 constexpr int kM2LGroupMax = 8;
 constexpr int m2lGroupSize(int L) { return L >= 8 ? 1 : L == 7 ? 3 : 4; }
 
