@@ -71,22 +71,18 @@ def log(msg):
 
 
 def m2l_nr_per_launch(L, mixed):
-    """Right-hand sides one M2L launch serves (the executor's rule: at most 16
-    double or 32 float complex accumulators per thread; 1 in double from
-    order 7, 2 in float at order 7; from order 8 a thread holds a column of
-    2L - 1 frequencies: 1 in double, 2 in float)."""
-    PP = (2 * L - 1) ** 3
-    if L >= 8:  # one column of 2L - 1 frequencies per thread
-        return 2 if mixed else 1
-    nw = max(-(-PP // 1024), min(-(-PP // 256), 3))
-    g = 3 if L == 7 else 4
-    cap = (32 if mixed else 16) // (g * nw)
-    w = 8 if cap >= 8 else 4 if cap >= 4 else 2 if cap >= 2 else 1
-    if not mixed and L >= 7:
+    """Right-hand sides that share one read of a table row in M2L (the
+    executor's rule: at most 16 double or 32 float complex accumulators per
+    thread, less where that spills; a launch of the stored variant covers up
+    to 8 such chunks one after another)."""
+    if mixed:
+        return 4 if L <= 4 else 2
+    if L >= 7:
         return 1
-    if L == 7 and w > 2:
-        return 2
-    return w
+    PP = (2 * L - 1) ** 3
+    nw = max(-(-PP // 1024), min(-(-PP // 256), 3))
+    cap = 16 // (4 * nw)
+    return 4 if cap >= 4 else 2 if cap >= 2 else 1
 
 
 def m2l_compulsory_bytes(st, L, nrhs, mixed, batched=False):
@@ -256,8 +252,9 @@ class Runner:
         flops = st["p2p_pairs"] * P2P_FLOPS_PER_PAIR * nrhs
         peak = PEAK_FP32_TFLOPS if mixed else PEAK_FP64_TFLOPS
         achieved = flops / t / 1e12
-        return {"kernel": "k_p2p + k_p2p_reduce", "bound": "valu", "achieved": achieved,
-                "peak": peak, "unit": "TFLOP/s", "frac": achieved / peak, "traffic": None,
+        return {"kernel": "k_p2p_lane or k_p2p_mfma, with k_p2p_reduce", "bound": "valu",
+                "achieved": achieved, "peak": peak, "unit": "TFLOP/s",
+                "frac": achieved / peak, "traffic": None,
                 "algorithmic_flops": flops, "avg_ms": stage_ms[dom]}
 
     def close(self):

@@ -15,7 +15,7 @@ under profiles/.
       per-kernel instruction counters (VALU, MFMA) and matrix-core busy
       fraction of one --pmc run
 
-A pass is the run of dispatches from one k_zero of the potentials (the
+A pass is the run of dispatches from one k_gather of the charges (the
 executor's first launch of a pass) to the next.  Its M2L stage is every
 k_m2l* launch, plus its k_m2f launches when the batched variant interleaves
 them with the M2L launches (a k_m2f after the first k_m2l of the pass).
@@ -64,6 +64,8 @@ def dispatches(path, counter=None):
         else:
             v = float(r["End_Timestamp"]) - float(r["Start_Timestamp"])
         grid = r.get("Grid_Size") or r.get("Grid_Size_X") or ""
+        if r.get("Grid_Size_Y"):  # (kernel traces give the sizes per dimension)
+            grid = str(int(grid) * int(r["Grid_Size_Y"]))
         out.append((int(r["Dispatch_Id"]), short(r["Kernel_Name"]), v, grid))
     out.sort()
     return out
@@ -75,22 +77,31 @@ def is_m2l(k):
 
 def passes(ds):
     """Split dispatches into evaluation passes; returns (start index, list)."""
-    cuts = [i for i, d in enumerate(ds) if d[1].startswith("dfm::k_zero<")]
+    cuts = [i for i, d in enumerate(ds) if d[1].startswith("dfm::k_gather")]
     out = []
     for a, b in zip(cuts, cuts[1:] + [len(ds)]):
         seg = ds[a:b]
-        # a pass ends with its scatters: drop whatever follows the last one
+        # a pass ends with its scatter: drop whatever follows
         last = max((i for i, d in enumerate(seg) if d[1].startswith("dfm::k_scatter")),
                    default=len(seg) - 1)
         out.append((a, seg[:last + 1]))
-    return out
+    # right-hand sides of each pass: its gather's work-items over those of the
+    # last pass of one (the first of a workload: a smaller or larger gather
+    # than a multiple of it starts the next workload)
+    widths, unit = [], 0
+    for _, seg in out:
+        g = int(seg[0][3])
+        if not unit or g % unit or g // unit > 64:
+            unit = g
+        widths.append(g // unit)
+    return [(a, seg, w) for (a, seg), w in zip(out, widths)]
 
 
-def describe(seg):
+def describe(seg, width):
     names = [d[1] for d in seg]
     m2l = [i for i, k in enumerate(names) if is_m2l(k)]
     prec = "f32" if any("<float" in k for k in names if is_m2l(k)) else "f64"
-    nrhs = sum(1 for k in names if k.startswith("dfm::k_gather"))
+    nrhs = width
     if not m2l:
         return prec, nrhs, "none", []
     first = m2l[0]
@@ -127,9 +138,9 @@ def cmd_traffic(a):
         keys = {}
         out.append("pass  prec  rhs  M2L variant  M2L launches  read GB  write GB  "
                    "(whole pass: read GB, write GB)")
-        for n, (s0, seg) in enumerate(passes(f[lo:hi])):
+        for n, (s0, seg, width) in enumerate(passes(f[lo:hi])):
             wseg = w[lo + s0: lo + s0 + len(seg)]
-            prec, nrhs, var, stage = describe(seg)
+            prec, nrhs, var, stage = describe(seg, width)
             rd = sum(seg[i][2] for i in stage) * 1024 * ff
             wr = sum(wseg[i][2] for i in stage) * 1024 * fw
             prd = sum(d[2] for d in seg) * 1024 * ff
@@ -182,8 +193,8 @@ def cmd_kernels(a):
             "durations) and of the whole pass:", "",
             "pass  prec  rhs  M2L variant  M2L launches  avg M2L launch us  M2L stage ms  "
             "pass kernels ms"]
-    for n, (s0, seg) in enumerate(passes(ds)):
-        prec, nrhs, var, stage = describe(seg)
+    for n, (s0, seg, width) in enumerate(passes(ds)):
+        prec, nrhs, var, stage = describe(seg, width)
         m2l = [seg[i][2] for i in stage if is_m2l(seg[i][1])]
         tot = sum(seg[i][2] for i in stage)
         avg = sum(m2l) / len(m2l) / 1e3 if m2l else 0.0
