@@ -730,15 +730,19 @@ static const int kVariantOfSigma[8] = {0, 1, 0, 2, 3, 0, 4, 5};
 // (100,000-point ellipsoid, order 6), at 1.95 to 2.40 (20,000-point cube,
 // order 8) and at 16.6 to 19.3 (1,000,000-point sphere, order 7).  With 8 they
 // end within 5% of one another: 1.43 -> 1.31, 2.39 -> 2.20 and 18.9 -> 17.6 ms
-// (4: 2.26 and 17.8; 16: 2.29 and 17.9).
+// (4: 2.26 and 17.8; 16: 2.29 and 17.9).  Short lists gain nothing and lose
+// rows shared across the cuts: 12,682 groups (30,000-point sphere, order 6)
+// 1.48 ms in one segment, 1.58 in eight, 5,666 groups 0.22 and 0.26, 7,800
+// groups a batch (cube, 16 right-hand sides) 24.1 and 24.4; from 1,024 groups a
+// part on the two are level or better.
 //
 // A launch covers up to kXcdChunks chunks of right-hand sides, chunk after
 // chunk; XCD x takes parts (x + chunk) mod 8, so that what still differs
 // between the parts evens out, and one chunk's tail overlaps the next's start:
 // 16 right-hand sides, ellipsoid 10.5 -> 9.8 ms, cube at order 4 1.28 -> 1.17,
 // at order 8 15.9 -> 15.5 (a launch per chunk before).
-constexpr int kXcdSegments = 8;      // at most
-constexpr int kXcdPartGroups = 128;  // groups of a part, at least (on average)
+constexpr int kXcdSegments = 8;       // at most
+constexpr int kXcdPartGroups = 1024;  // groups of a part, at least (on average)
 constexpr int kXcdChunks = 8;
 struct XcdParts {
   int segments, chunks;
