@@ -22,6 +22,7 @@
 #include "grid.hpp"
 #include "dft.hpp"
 #include "kernels.hpp"
+#include "leaf_items.hpp"
 #include "leaf_slots.hpp"
 #include "p2p.hpp"
 #include "plan.hpp"
@@ -206,7 +207,7 @@ __global__ __launch_bounds__(128) void k_p2m(const int2* __restrict__ items, Dev
 // covers whole 128-byte lines (with the operands the other way round, 8 bytes
 // of every 32; that and four steps a time instead of one: 100,000-point
 // ellipsoid, order 6, 2.36 -> 1.95 ms, 20,000-point cube, order 8, 2.37 -> 1.66).
-constexpr int kP2MMfmaNR = 16, kP2MMfmaSlots = 32, kP2MMfmaPoints = 64;
+constexpr int kP2MMfmaNR = 16;
 template <int L>
 __global__ __launch_bounds__(256) void k_p2m_mfma(
     const int2* __restrict__ items, DevCells S, DevLevels lv, const double* __restrict__ px,
@@ -2355,37 +2356,18 @@ static int upload(Exec& X, Plan& pl) {
   CKR(X.upv(X.perm, pl.perm));
   CKR(X.upv(X.p2m, pl.p2mCell)); X.np2m = (int)pl.p2mCell.size();
   {
-    // P2M work items: leaves with several slots on the matrix cores, the
-    // others in passes of p2mSlotsPerPass(L) slots
-    const int C = p2mSlotsPerPass(pl.L);
-    std::vector<int2> it, slots, mf, big, bigSlots;
-    for (int c : pl.p2mCell) {
-      const int nsl = std::max(1, pl.S.nslot[c]);
-      const bool small = pl.S.nprt[c] <= kP2MMfmaPoints;
-      if (nsl >= p2mSlotsMin(pl.p2mCell.size())) {
-        for (int k0 = 0; k0 < nsl; k0 += kSlotCols) {
-          slots.push_back(make_int2(c, k0));
-          if (!small) bigSlots.push_back(make_int2(c, k0));
-        }
-      } else {
-        for (int k0 = 0; k0 < nsl; k0 += C) {
-          it.push_back(make_int2(c, k0));
-          if (!small) big.push_back(make_int2(c, k0));
-        }
-      }
-      if (small)
-        for (int k0 = 0; k0 < nsl; k0 += kP2MMfmaSlots) mf.push_back(make_int2(c, k0));
-    }
-    CKR(X.upv(X.p2mItems, it));
-    X.np2mItems = (int)it.size();
-    CKR(X.upv(X.p2mSlotItems, slots));
-    X.np2mSlot = (int)slots.size();
-    CKR(X.upv(X.p2mMfmaItems, mf));
-    X.np2mMfma = (int)mf.size();
-    CKR(X.upv(X.p2mBigItems, big));
-    X.np2mBig = (int)big.size();
-    CKR(X.upv(X.p2mBigSlotItems, bigSlots));
-    X.np2mBigSlot = (int)bigSlots.size();
+    P2MItems<int2> it;
+    buildP2MItems(pl, p2mSlotsPerPass(pl.L), it);
+    CKR(X.upv(X.p2mItems, it.few));
+    X.np2mItems = (int)it.few.size();
+    CKR(X.upv(X.p2mSlotItems, it.slots));
+    X.np2mSlot = (int)it.slots.size();
+    CKR(X.upv(X.p2mMfmaItems, it.mfma));
+    X.np2mMfma = (int)it.mfma.size();
+    CKR(X.upv(X.p2mBigItems, it.bigFew));
+    X.np2mBig = (int)it.bigFew.size();
+    CKR(X.upv(X.p2mBigSlotItems, it.bigSlots));
+    X.np2mBigSlot = (int)it.bigSlots.size();
   }
   {
     // L2P leaves of few slots (k_l2p); the others are cut into items at the

@@ -13,20 +13,10 @@
 #include <hip/hip_runtime.h>
 
 #include "kernels.hpp"
+#include "leaf_items.hpp"
 
 namespace dfm {
 
-constexpr int kSlotCols = 16;    // slots per matrix-core tile
-// Leaves with fewer slots stay on the vector units, whose work does not round
-// slots up to 16: L2P of a million points at 16 wavelengths, 17 slots a leaf,
-// takes 1.5 ms with a line at 24 and 2.3 with one at 6 (order 7, float), at 50
-// slots a leaf (41,334 points, order 6, double) 0.28 against 0.49; P2M, whose
-// vector kernel is further behind, gains from 6 slots on (1.19 -> 0.91 ms).
-// Plans of few leaves leave SIMDs idle on either path, so rounding up costs
-// nothing there, splitting a leaf's slots over blocks pays (510 leaves, order
-// 10: L2P 0.61 -> 0.42 ms with the line at 6), and one kernel does for all.
-inline int p2mSlotsMin(size_t leaves) { return leaves < 2048 ? 1 : 6; }
-inline int l2pSlotsMin(size_t leaves) { return leaves < 2048 ? 1 : 24; }
 constexpr int kL2PSlots = 128;   // slots per block of k_l2p_slots
 
 typedef double mfma_v4d __attribute__((ext_vector_type(4)));
@@ -97,6 +87,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(3))) void k_
   const int2 it = items[item];
   const int c = it.x, k0 = it.y;
   const int lvl = S.lvl[c], pb = S.pbeg[c], n = S.nprt[c], s0 = S.slot0[c], ns = S.nslot[c];
+  if (k0 >= ns) return;  // (ns - 1 below is one of the leaf's slots)
   const double ctr[3] = {S.ctr[3 * c], S.ctr[3 * c + 1], S.ctr[3 * c + 2]}, rad = S.rad[c];
   const int hf = lv.isHF[lvl], doff = lv.dirOff[lvl], srow = lv.sigRow0[lvl];
   const int lane = threadIdx.x;
