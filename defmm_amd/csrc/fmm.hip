@@ -24,6 +24,7 @@
 #include "kernels.hpp"
 #include "leaf_items.hpp"
 #include "leaf_slots.hpp"
+#include "near_items.hpp"
 #include "p2p.hpp"
 #include "plan.hpp"
 #include "xfer.hpp"
@@ -2239,62 +2240,6 @@ static int reupload(Exec& X, int oldNr, int oldPrec, int oldMode, bool oldAuto, 
   return rc;
 }
 
-// Near-field items: a leaf's targets in chunks of at most tg (p2pChunk), its
-// source list in equal runs (multiples of 64) of at most `budget` sources.
-// 8,192 sources a run amortise a wave's start and final sums; where that
-// leaves fewer than 16,384 items (16 waves per SIMD's share of the chip are
-// needed to hide latency and even out the end) the budget is halved, down to
-// 512.
-static int buildP2PItems(const Plan& pl, int tg, std::vector<P2PItem>& items,
-                         std::vector<int>& beg) {
-  const Tree& T = pl.T;
-  const size_t nl = pl.p2pLeaf.size();
-  std::vector<int64_t> total(nl, 0);
-  for (size_t lf = 0; lf < nl; lf++)
-    for (int r = pl.p2pBeg[lf]; r < pl.p2pBeg[lf + 1]; r++)
-      total[lf] += pl.p2pSrcE[r] - pl.p2pSrcB[r];
-  auto chunksOf = [&](size_t lf) { return (T.nprt[pl.p2pLeaf[lf]] + tg - 1) / tg; };
-  int64_t budget = 8192;
-  for (;; budget /= 2) {
-    int64_t n = 0;
-    for (size_t lf = 0; lf < nl; lf++) n += chunksOf(lf) * ((total[lf] + budget - 1) / budget);
-    if (n > INT32_MAX / 2) {
-      g_err = "near-field work items exceed the launch index range";
-      return ERR_ARG;
-    }
-    if (n >= 16384 || budget <= 512) {
-      items.reserve((size_t)n);
-      break;
-    }
-  }
-  for (size_t lf = 0; lf < nl; lf++) {
-    beg.push_back((int)items.size());
-    const int n = T.nprt[pl.p2pLeaf[lf]], chunks = chunksOf(lf);
-    const int64_t runs = (total[lf] + budget - 1) / budget;
-    if (runs == 0 || chunks == 0) continue;
-    const int chunk = p2pChunk(n, tg);
-    const int64_t len = ((total[lf] + runs - 1) / runs + 63) / 64 * 64;
-    int r = pl.p2pBeg[lf], off = 0;
-    for (int64_t pos = 0; pos < total[lf]; pos += len) {
-      const int cnt = (int)std::min(len, total[lf] - pos);
-      while (off >= pl.p2pSrcE[r] - pl.p2pSrcB[r]) {
-        off -= pl.p2pSrcE[r] - pl.p2pSrcB[r];
-        r++;
-      }
-      for (int t0 = 0; t0 < n; t0 += chunk)
-        items.push_back({(int)lf, t0, std::min(chunk, n - t0), r, off, cnt});
-      off += cnt;
-    }
-    // the reduction counts ceil(n / tg) items per run
-    if (((int)items.size() - beg.back()) % chunks != 0) {
-      g_err = "internal: near-field items do not match the leaf's chunks";
-      return ERR_STATE;
-    }
-  }
-  beg.push_back((int)items.size());
-  return OK;
-}
-
 static int upload(Exec& X, Plan& pl) {
   X.L = pl.L; X.P = pl.P; X.LL = pl.LL; X.PP = pl.PP; X.kappa = pl.kappa;
   {
@@ -2484,20 +2429,16 @@ static int upload(Exec& X, Plan& pl) {
   X.hGSrcF.swap(pl.m2lGSrcF);
   X.hM2fSlot = pl.m2fSlot;
   X.hGroupBeg = pl.m2lGroupBeg;
-  // P2P work items: 64-target chunks x runs of <= budget sources.  The
-  // budget is 4,096 sources unless that leaves fewer than 16,384 items (too
-  // few waves to fill 1,024 SIMDs: the 20,000-point cube has 3,249); then it
-  // is halved, down to 512.
   {
     std::vector<P2PItem> items;
     std::vector<int> beg;
-    CKR(buildP2PItems(pl, kP2PTargets, items, beg));
+    CKR(buildP2PItems(pl, kP2PTargets, items, beg, g_err));
     X.nLaneItems = (int)items.size();
     CKR(X.upv(X.laneItems, items));
     CKR(X.upv(X.laneItemBeg, beg));
     items.clear();
     beg.clear();
-    CKR(buildP2PItems(pl, kP2PMfmaTargets, items, beg));
+    CKR(buildP2PItems(pl, kP2PMfmaTargets, items, beg, g_err));
     X.nitems = (int)items.size();
     X.nleaves = (int)pl.p2pLeaf.size();
     X.st.p2p_items = X.nitems;

@@ -9,6 +9,7 @@
 #include <hip/hip_runtime.h>
 
 #include "kernels.hpp"
+#include "near_items.hpp"
 #include "phase.hpp"
 
 namespace dfm {
@@ -53,21 +54,6 @@ __device__ __forceinline__ void p2pValue(double x, double y, double z, const Pha
     co *= K;
     si *= K;
   }
-}
-
-// Work item: nt targets of one leaf, from t0 (leaf-relative), against cnt
-// sources of its list from (range r, offset off).
-struct P2PItem {
-  int leaf, t0, nt, r, off, cnt;
-};
-// Targets per item of k_p2p_lane, at most.
-constexpr int kP2PTargets = 8;
-// A leaf's n targets are cut into equal chunks of at most tg; tg itself where
-// an item works on whole row blocks of 16.
-DFM_HD inline int p2pChunk(int n, int tg) {
-  if (tg % 16 == 0) return tg;
-  const int chunks = (n + tg - 1) / tg;
-  return (n + chunks - 1) / chunks;
 }
 
 // Sum of v over the wave, N values (a power of two, at most 64) at once: each
@@ -279,7 +265,7 @@ __global__ __launch_bounds__(256) void k_p2p_lane(
 // sources and polynomials of kappa r over [-pi/4, pi/4], took 5.2 ms where
 // this takes 4.0 (100,000-point ellipsoid at 64 wavelengths, Ncrit 97) and
 // 1.07 for 0.74 (20,000-point cube).
-constexpr int kP2PMfmaNR = 16, kP2PMfmaTargets = 32;
+constexpr int kP2PMfmaNR = 16;
 struct P2PMfmaArgs {
   const P2PItem* items;
   const int *leafCell, *tpbeg;
