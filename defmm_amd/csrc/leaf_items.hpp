@@ -1,5 +1,6 @@
-// Work items of P2M, built at upload.  Host-only and free of HIP types, so
-// that a plain C++ program can check them (HIP sources read them as int2).
+// Rules and work items of the leaves' operators, used at upload.  Free of HIP
+// types, so that a plain C++ program can check them (HIP sources read the
+// items as int2).
 #pragma once
 #include <algorithm>
 #include <vector>
@@ -19,6 +20,15 @@ constexpr int kSlotCols = 16;    // slots per matrix-core tile (leaf_slots.hpp)
 // 10: L2P 0.61 -> 0.42 ms with the line at 6), and one kernel does for all.
 inline int p2mSlotsMin(size_t leaves) { return leaves < 2048 ? 1 : 6; }
 inline int l2pSlotsMin(size_t leaves) { return leaves < 2048 ? 1 : 24; }
+
+// Matrix-core steps (of 4 weight indices) of k_l2p_slots whose sum is added to
+// the slot's: one chain of L^3 terms is less exact than the vector kernel's
+// nested sums of L and L^2 (float, random coefficients, order 8: 4.0e-7 and
+// 1.6e-7, in chains of 16 terms 1.3e-7; order 4: 1.5e-7 and 8.6e-8, in chains
+// of 8 terms 8.4e-8).  Far field of 40,000 points on a sphere at 24
+// wavelengths, float, order 6: relative error 5.2e-7 with one chain, 4.6e-7
+// with these, 4.8e-7 with the vector kernel.
+constexpr int l2pSlotChain(int L) { return L <= 4 ? 2 : 4; }
 
 // P2M for 16 right-hand sides: slots per block, points of a leaf at most
 constexpr int kP2MMfmaSlots = 32, kP2MMfmaPoints = 64;

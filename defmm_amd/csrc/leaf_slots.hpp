@@ -195,8 +195,9 @@ struct L2PItem {
 // Bound by reading the expansions (as much as P2M writes) and by the loads'
 // latency.  Against lanes per point reading the slots' rows from LDS (k_l2p),
 // a block per leaf whatever its number of slots: 20,000 points order 8 0.75 ->
-// 0.32 ms (double), 0.44 -> 0.22 ms (float), 200,000-point sphere order 5 3.7
-// -> 2.3 ms (double).
+// 0.31 ms (double), 0.44 -> 0.22 ms (float), 200,000-point sphere order 5 3.7
+// -> 2.3 ms (double).  Adding the chains up (l2pSlotChain) costs 5% at orders
+// 5 and 6 (41,334 points, double, 0.30 -> 0.32 ms) and nothing at 7 and 8.
 template <typename R, int L>
 __global__ __launch_bounds__(256) void k_l2p_slots(
     const L2PItem* __restrict__ items, DevCells T, DevLevels lv, const double* __restrict__ px,
@@ -208,6 +209,8 @@ __global__ __launch_bounds__(256) void k_l2p_slots(
   typedef Mfma16<R> X;
   constexpr int LL = L * L * L, KS = (LL + 3) / 4, TP = l2pSlotTile<R, L>(), NB = TP / 16;
   constexpr int ST = l2pSlotStride<R, L>(), kU = sizeof(R) == 8 ? 4 : 8;
+  constexpr int kB = l2pSlotChain(L);
+  static_assert(kU % kB == 0, "chains end with a batch of loads");
   static_assert(ST >= 4 * KS, "rows of S hold the last step's padding");
   __shared__ R Sm[TP][ST];
   __shared__ R Wt[3][TP][L];
@@ -254,6 +257,8 @@ __global__ __launch_bounds__(256) void k_l2p_slots(
       cre[b] = typename X::V{0, 0, 0, 0};
       cim[b] = typename X::V{0, 0, 0, 0};
     }
+    // (not unrolled: the loads of the batches to come would fill the registers)
+#pragma unroll 1
     for (int ks0 = 0; ks0 < KS; ks0 += kU) {
       R2 lv2[kU], sv[kU];
 #pragma unroll
@@ -264,15 +269,27 @@ __global__ __launch_bounds__(256) void k_l2p_slots(
       }
       __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-      for (int u = 0; u < kU; u++) {
-        if (ks0 + u >= KS) break;
-        const int kk = 4 * (ks0 + u) + quad;
-        const R2 bv = hf ? cmul(lv2[u], sv[u]) : lv2[u];
+      for (int u0 = 0; u0 < kU; u0 += kB) {
+        if (ks0 + u0 >= KS) break;
+        typename X::V tre[NB], tim[NB];
+#pragma unroll
+        for (int b = 0; b < NB; b++) tre[b] = tim[b] = typename X::V{0, 0, 0, 0};
+#pragma unroll
+        for (int u = u0; u < u0 + kB; u++) {
+          if (ks0 + u >= KS) break;
+          const int kk = 4 * (ks0 + u) + quad;
+          const R2 bv = hf ? cmul(lv2[u], sv[u]) : lv2[u];
+#pragma unroll
+          for (int b = 0; b < NB; b++) {
+            const R a = Sm[16 * b + lr][kk];
+            tre[b] = X::mac(a, bv.x, tre[b]);
+            tim[b] = X::mac(a, bv.y, tim[b]);
+          }
+        }
 #pragma unroll
         for (int b = 0; b < NB; b++) {
-          const R a = Sm[16 * b + lr][kk];
-          cre[b] = X::mac(a, bv.x, cre[b]);
-          cim[b] = X::mac(a, bv.y, cim[b]);
+          cre[b] += tre[b];
+          cim[b] += tim[b];
         }
       }
     }
