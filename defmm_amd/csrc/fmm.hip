@@ -1771,7 +1771,7 @@ struct Exec {
   void* Lb = nullptr;        // local expansions (aliases ML when F is stored)
   size_t mStride = 0, lStride = 0, fStride = 0;  // elements between right-hand sides
   int m2lMode = DEFMM_M2L_STORED;
-  bool p2pMfma = true;       // float P2P in chunks of 16 right-hand sides on the matrix cores
+  bool p2pMfma = true;       // float P2P in chunks of 16 or 8 right-hand sides on the matrix cores
   bool m2lAuto = true;       // mode chosen by free memory (until set explicitly)
   int nr = 1;                // right-hand sides the expansion stores hold
   int batchRows = 16384;     // requested workspace rows of the batched M2L
@@ -2002,8 +2002,8 @@ __global__ void k_table_rows(const int* __restrict__ keys, int64_t nrows,
 // pass of X.nr right-hand sides uses.
 static size_t partialElems(const Exec& X) {
   size_t n = (size_t)X.nLaneItems * std::min(X.nr, X.prec == DEFMM_MIXED ? 8 : 4) * kP2PTargets;
-  if (X.prec == DEFMM_MIXED && X.nr >= kP2PMfmaNR)
-    n = std::max(n, (size_t)X.nitems * kP2PMfmaTargets * kP2PMfmaNR);
+  if (X.prec == DEFMM_MIXED && X.nr >= 8)
+    n = std::max(n, (size_t)X.nitems * kP2PMfmaTargets * (X.nr >= kP2PMfmaNR ? kP2PMfmaNR : 8));
   return std::max<size_t>(n, 1);
 }
 
@@ -2554,6 +2554,7 @@ static void launchP2PLane(Exec& X, hipStream_t s, int r0) {
 }
 
 // 16 right-hand sides r0 .. r0 + 15 of the float path on the matrix cores
+template <int NR>
 static void launchP2PMfma(Exec& X, hipStream_t s, int r0) {
   const float2* q = (const float2*)X.q + (size_t)r0 * X.ns;
   float2* p = (float2*)X.p + (size_t)r0 * X.nt;
@@ -2561,13 +2562,13 @@ static void launchP2PMfma(Exec& X, hipStream_t s, int r0) {
                          (size_t)X.ns, X.rb, X.re, (const float2*)X.phaseTab, X.partial,
                          X.nitems};
   auto go = [&](auto phase) {
-    hipLaunchKernelGGL((k_p2p_mfma<decltype(phase)::value>),
+    hipLaunchKernelGGL((k_p2p_mfma<decltype(phase)::value, NR>),
                        itemGrid(((int64_t)X.nitems + 3) / 4), dim3(256), 0, s, A, X.phaseConsts);
   };
   if (X.p2pPhase == kPhaseNone) go(std::integral_constant<int, kPhaseNone>());
   else if (X.p2pPhase == kPhaseTable) go(std::integral_constant<int, kPhaseTable>());
   else go(std::integral_constant<int, kPhaseLibrary>());
-  hipLaunchKernelGGL((k_p2p_reduce<float, kP2PMfmaNR, kP2PMfmaTargets>), itemGrid(X.nleaves),
+  hipLaunchKernelGGL((k_p2p_reduce<float, NR, kP2PMfmaTargets>), itemGrid(X.nleaves),
                      dim3(256), 0, s, X.itemBeg, X.leafCell, X.T.pbeg, X.T.nprt,
                      (const double2*)X.partial, p, (size_t)X.nt, X.nleaves);
 }
@@ -2575,8 +2576,8 @@ static void launchP2PMfma(Exec& X, hipStream_t s, int r0) {
 // One evaluation pass for nrhs <= X.nr right-hand sides: qin / pout hold
 // nrhs x n complex128 values, right-hand side after right-hand side, in
 // input order.  Stages as in the reference's gemv.  P2M, L2P and P2P go by
-// groups of right-hand sides (16 on the matrix cores in float; P2P up to 8
-// per kernel value otherwise, P2M and L2P one), M2L by m2lLaunch, the other
+// groups of right-hand sides (16 on the matrix cores in float; P2P 8 there, up
+// to 4 per kernel value otherwise, P2M and L2P one), M2L by m2lLaunch, the other
 // stages take all in one launch.
 template <typename R, int L>
 static int runTyped(Exec& X, const double2* qin, double2* pout, int parts, int nrhs,
@@ -2745,16 +2746,20 @@ static int runTyped(Exec& X, const double2* qin, double2* pout, int parts, int n
     }
   mark(7);
   if (near && X.nitems) {
-    // near field: per-item partial sums, then folded into p per target leaf,
-    // up to 8 right-hand sides per kernel value on the VALU (double: 4, whose
-    // sums fit the registers; two launches of 4 take 1.02 ms at 20,000 points
-    // where one of 8 took 1.41), 16 on the matrix cores in float.  (Run on a second stream beside M2L it measured
-    // no faster: both contend for the same CUs.)
+    // near field: per-item partial sums, then folded into p per target leaf;
+    // in float 16 or 8 right-hand sides per kernel value on the matrix cores,
+    // otherwise up to 8 on the VALU (double: 4, whose sums fit the registers;
+    // two launches of 4 take 1.02 ms at 20,000 points where one of 8 took
+    // 1.41).  (Run on a second stream beside M2L it measured no faster: both
+    // contend for the same CUs.)
     for (int r0 = 0; r0 < nrhs;) {
       const int n = nrhs - r0;
       if (sizeof(R) == 4 && n >= kP2PMfmaNR && X.p2pMfma) {
-        launchP2PMfma(X, s, r0);
+        launchP2PMfma<kP2PMfmaNR>(X, s, r0);
         r0 += kP2PMfmaNR;
+      } else if (sizeof(R) == 4 && n >= 8 && X.p2pMfma) {
+        launchP2PMfma<8>(X, s, r0);
+        r0 += 8;
       } else if (sizeof(R) == 4 && n >= 8) { launchP2PLane<R, 8>(X, s, r0); r0 += 8; }
       else if (n >= 4) { launchP2PLane<R, 4>(X, s, r0); r0 += 4; }
       else if (n == 3) { launchP2PLane<R, 3>(X, s, r0); r0 += 3; }

@@ -1,5 +1,5 @@
 // Near field: with a lane per source (1, 2, 3, 4 or 8 right-hand sides), and
-// on the matrix cores (16, float).
+// on the matrix cores (16 or 8, float).
 //
 //   p_i += sum_j exp(i kappa r) / (4 pi r) q_j,  r = |x_i - y_j|,
 // term 0 when r^2 < 1e-16 (reference include/operators/P2P.hpp:42-79).
@@ -103,7 +103,8 @@ __device__ __forceinline__ int waveSumIndex(int lane) {
 // sphere at 64 wavelengths (8.67e9 pairs): double 23.8 -> 13.2 ms, float
 // 14.5 -> 8.6 ms; 4,000-point cube 80 -> 27 us; 150,000-point Laplace
 // clusters (no phase) 0.85 -> 0.27 ms; 20,000-point cube, float: 2 right-hand
-// sides 0.50 -> 0.31 ms, 3: 0.90 -> 0.34, 4: 0.53 -> 0.40, 8: 0.73 -> 0.74.
+// sides 0.50 -> 0.31 ms, 3: 0.90 -> 0.34, 4: 0.53 -> 0.40 (8, where the matrix
+// cores are switched off: 0.73 -> 0.74).
 // TC targets per sweep of the sources keep the accumulators in registers.
 constexpr int kP2PFlush = 16;
 template <typename R, int NR>
@@ -239,16 +240,19 @@ __global__ __launch_bounds__(256) void k_p2p_lane(
   }
 }
 
-// 16 right-hand sides of the float path on the matrix cores.  An item's sums
-// are the product of the kernel matrix G (targets x sources, complex, one
+// 16 or 8 right-hand sides of the float path on the matrix cores.  An item's
+// sums are the product of the kernel matrix G (targets x sources, complex, one
 // element per lane and step, phase reduced in double) and the charges Q
-// (sources x 16):
+// (sources x right-hand sides):
 //   P_re += G_re Q_re - G_im Q_im,   P_im += G_re Q_im + G_im Q_re,
-// four V_MFMA_F32_16X16X4_F32 per 4 sources and 16 targets.  Operands: A (16
-// x 4) lane l holds row l % 16, column l / 16; B (4 x 16) row l / 16, column
+// V_MFMA_F32_16X16X4_F32s of 4 sources and 16 targets.  Operands: A (16 x 4)
+// lane l holds row l % 16, column l / 16; B (4 x 16) row l / 16, column
 // l % 16; D (16 x 16) column l % 16, rows 4 (l / 16) + 0..3.  So lane l
 // evaluates G for target l % 16 of a row block and source 4 k + l / 16 of
-// step k, and ends with right-hand side l % 16 of targets 4 (l / 16) + 0..3.
+// step k.  16 right-hand sides take four of them a step (P_re and P_im apart,
+// a column each); 8 take two, with the columns of Q_re | Q_im against G_re and
+// of -Q_im | Q_re against G_im, so that P_re and P_im are the two halves of
+// one result.  Lane l ends with column l % 16 of targets 4 (l / 16) + 0..3.
 //
 // A wave per item of at most kP2PMfmaTargets targets (two row blocks, which
 // share the source operands), 4 items per block with the phase table in LDS.
@@ -257,14 +261,19 @@ __global__ __launch_bounds__(256) void k_p2p_lane(
 // ahead; no barrier, so no wave waits for another.  Every 64 sources the sums
 // are added to double ones.
 //
-// Bound by the SIMD's issue: 64 pairs take the matrix core 128 clocks and the
-// vector unit about 200 (34 instructions, 16 of them double), and on this chip
-// the two do not overlap, not even between waves (four waves of
-// V_MFMA_F32_16X16X4_F32 and 8 independent v_fma each: 74 clocks, 35 and 36
-// alone).  A block of 4 waves per 64 targets, with three barriers per 64
-// sources and polynomials of kappa r over [-pi/4, pi/4], took 5.2 ms where
-// this takes 4.0 (100,000-point ellipsoid at 64 wavelengths, Ncrit 97) and
-// 1.07 for 0.74 (20,000-point cube).
+// Bound by the SIMD's issue: 64 pairs take the matrix core 128 clocks (16
+// right-hand sides; 64 for 8) and the vector unit about 200 (34 instructions,
+// 16 of them double), and on this chip the two do not overlap, not even
+// between waves (four waves of V_MFMA_F32_16X16X4_F32 and 8 independent v_fma
+// each: 74 clocks, 35 and 36 alone).  A block of 4 waves per 64 targets, with
+// three barriers per 64 sources and polynomials of kappa r over [-pi/4, pi/4],
+// took 5.2 ms where this takes 4.0 (100,000-point ellipsoid at 64 wavelengths,
+// Ncrit 97, 16 right-hand sides) and 1.07 for 0.74 (20,000-point cube).
+// 8 right-hand sides: 200,000-point sphere at 40 wavelengths 11.9 ms, with a
+// lane per source 19.9 (two targets a sweep are too few for each source's
+// loads), with a lane per target and polynomials 16.3; 100,000 clustered
+// points without phase 0.17, 0.52 and 0.43; 5,000-point cube 0.073, 0.086 and
+// 0.111.
 constexpr int kP2PMfmaNR = 16;
 struct P2PMfmaArgs {
   const P2PItem* items;
@@ -277,12 +286,14 @@ struct P2PMfmaArgs {
   double2* partial;
   int nItems;
 };
-// One item with MB row blocks; lc and lq are the wave's stage, tab the
-// block's phase table.
-template <int Phase, int MB>
+// One item of NR right-hand sides with MB row blocks; lc and lq are the wave's
+// stage, tab the block's phase table.  lq[source][column]: the charge (16), or
+// the operands (Q_re, -Q_im) and (Q_im, Q_re) of columns r and r + 8 (8).
+template <int Phase, int NR, int MB>
 __device__ __forceinline__ void p2pMfmaItem(const P2PMfmaArgs& A, const PhaseConsts& pc, int item,
                                             const P2PItem& it, const float2* tab,
-                                            double (*lc)[16], float2 (*lq)[kP2PMfmaNR + 1]) {
+                                            double (*lc)[16], float2 (*lq)[17]) {
+  static_assert(NR == 16 || NR == 8, "columns of the result");
   typedef float v4f __attribute__((ext_vector_type(4)));
   constexpr int kStage = 16;
   const int lane = threadIdx.x & 63, lr = lane & 15, kq = lane >> 4;
@@ -296,7 +307,7 @@ __device__ __forceinline__ void p2pMfmaItem(const P2PMfmaArgs& A, const PhaseCon
     yt[b] = A.ty[i];
     zt[b] = A.tz[i];
   }
-  v4f dre[MB], dim[MB];
+  v4f dre[MB], dim[MB];  // (dim, ai: of 16 right-hand sides)
   double ar[MB][4], ai[MB][4];
 #pragma unroll
   for (int b = 0; b < MB; b++) {
@@ -322,11 +333,11 @@ __device__ __forceinline__ void p2pMfmaItem(const P2PMfmaArgs& A, const PhaseCon
   const double* sc = kq == 0 ? A.sx : kq == 1 ? A.sy : A.sz;
   const float2* ql = A.q + (size_t)kq * A.qStride;
   double nc;
-  float2 nq[4];
+  float2 nq[NR / 4];
   auto load = [&]() {
     nc = sc[j];
 #pragma unroll
-    for (int u = 0; u < 4; u++) nq[u] = ql[4 * u * A.qStride + j];
+    for (int u = 0; u < NR / 4; u++) nq[u] = ql[4 * u * A.qStride + j];
   };
   advance(lr, lr);
   load();
@@ -338,7 +349,15 @@ __device__ __forceinline__ void p2pMfmaItem(const P2PMfmaArgs& A, const PhaseCon
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
     if (kq < 3) lc[kq][lr] = nc;
 #pragma unroll
-    for (int u = 0; u < 4; u++) lq[lr][kq + 4 * u] = valid ? nq[u] : make_float2(0.f, 0.f);
+    for (int u = 0; u < NR / 4; u++) {
+      const float2 c = valid ? nq[u] : make_float2(0.f, 0.f);
+      if constexpr (NR == 16) {
+        lq[lr][kq + 4 * u] = c;
+      } else {
+        lq[lr][kq + 4 * u] = make_float2(c.x, -c.y);
+        lq[lr][kq + 4 * u + 8] = make_float2(c.y, c.x);
+      }
+    }
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
     __builtin_amdgcn_wave_barrier();
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
@@ -349,16 +368,18 @@ __device__ __forceinline__ void p2pMfmaItem(const P2PMfmaArgs& A, const PhaseCon
       const int s = 4 * k + kq;
       const double xs = lc[0][s], ys = lc[1][s], zs = lc[2][s];
       const float2 ch = lq[s][lr];
-      const float mi = -ch.y;
+      const float im = NR == 16 ? -ch.y : ch.y;
 #pragma unroll
       for (int b = 0; b < MB; b++) {
         float co, si;
         p2pValue<Phase, float>(xt[b] - xs, yt[b] - ys, zt[b] - zs, pc, tab, co, si);
         dre[b] = __builtin_amdgcn_mfma_f32_16x16x4f32(co, ch.x, dre[b], 0, 0, 0);
-        dim[b] = __builtin_amdgcn_mfma_f32_16x16x4f32(co, ch.y, dim[b], 0, 0, 0);
+        if constexpr (NR == 16)
+          dim[b] = __builtin_amdgcn_mfma_f32_16x16x4f32(co, ch.y, dim[b], 0, 0, 0);
         if constexpr (Phase != kPhaseNone) {
-          dre[b] = __builtin_amdgcn_mfma_f32_16x16x4f32(si, mi, dre[b], 0, 0, 0);
-          dim[b] = __builtin_amdgcn_mfma_f32_16x16x4f32(si, ch.x, dim[b], 0, 0, 0);
+          dre[b] = __builtin_amdgcn_mfma_f32_16x16x4f32(si, im, dre[b], 0, 0, 0);
+          if constexpr (NR == 16)
+            dim[b] = __builtin_amdgcn_mfma_f32_16x16x4f32(si, ch.x, dim[b], 0, 0, 0);
         }
       }
     }
@@ -368,7 +389,7 @@ __device__ __forceinline__ void p2pMfmaItem(const P2PMfmaArgs& A, const PhaseCon
 #pragma unroll
         for (int v = 0; v < 4; v++) {
           ar[b][v] += (double)dre[b][v];
-          ai[b][v] += (double)dim[b][v];
+          if constexpr (NR == 16) ai[b][v] += (double)dim[b][v];
         }
         dre[b] = dim[b] = v4f{0.f, 0.f, 0.f, 0.f};
       }
@@ -380,18 +401,19 @@ __device__ __forceinline__ void p2pMfmaItem(const P2PMfmaArgs& A, const PhaseCon
 #pragma unroll
     for (int v = 0; v < 4; v++) {
       const int t = 16 * b + 4 * kq + v;
-      if (t < it.nt)
-        A.partial[((size_t)item * kP2PMfmaNR + lr) * kP2PMfmaTargets + t] =
-            make_double2(ar[b][v] * kInv4Pi, ai[b][v] * kInv4Pi);
+      if (t >= it.nt) continue;
+      double2* o = A.partial + ((size_t)item * NR + lr % NR) * kP2PMfmaTargets + t;
+      if constexpr (NR == 16) *o = make_double2(ar[b][v] * kInv4Pi, ai[b][v] * kInv4Pi);
+      else ((double*)o)[lr / NR] = ar[b][v] * kInv4Pi;
     }
 }
 // (at least 4 waves per SIMD: the sums then stay in registers that both kinds
 // of instruction take)
-template <int Phase>
+template <int Phase, int NR>
 __global__ __launch_bounds__(256, 4) void k_p2p_mfma(P2PMfmaArgs A, PhaseConsts pc) {
   __shared__ float2 tab[Phase == kPhaseTable ? kPhaseN : 1];
   __shared__ double lc[4][3][16];
-  __shared__ float2 lq[4][16][kP2PMfmaNR + 1];
+  __shared__ float2 lq[4][16][17];
   if constexpr (Phase == kPhaseTable) {
     static_assert(kPhaseN == 256, "one table entry per thread");
     tab[threadIdx.x] = A.phase[threadIdx.x];
@@ -401,8 +423,8 @@ __global__ __launch_bounds__(256, 4) void k_p2p_mfma(P2PMfmaArgs A, PhaseConsts 
   const int item = (int)(blockIdx.y * gridDim.x + blockIdx.x) * 4 + w;
   if (item >= A.nItems) return;
   const P2PItem it = A.items[item];
-  if (it.nt > 16) p2pMfmaItem<Phase, 2>(A, pc, item, it, tab, lc[w], lq[w]);
-  else p2pMfmaItem<Phase, 1>(A, pc, item, it, tab, lc[w], lq[w]);
+  if (it.nt > 16) p2pMfmaItem<Phase, NR, 2>(A, pc, item, it, tab, lc[w], lq[w]);
+  else p2pMfmaItem<Phase, NR, 1>(A, pc, item, it, tab, lc[w], lq[w]);
 }
 
 // Adds the partial sums of a leaf's items to p: the leaf's targets are cut

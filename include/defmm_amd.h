@@ -224,13 +224,13 @@ int defmm_plan_set_memory_limit(defmm_plan plan, int64_t bytes);
 /*
  * Execution options of a plan (no reallocation; waits for the plan's last
  * execution).  DEFMM_OPT_P2P_MFMA: 1 (default) evaluates the near field of
- * the mixed-precision path 16 right-hand sides at a time on the matrix cores
- * when the plan's width allows it; 0 keeps it on the vector units (up to 8
- * right-hand sides per kernel value).  DEFMM_OPT_L2P_MFMA: the same for L2P
- * (1 by default: 16 right-hand sides per pass over a leaf's slots on the
- * matrix cores; 0: one right-hand side per pass on the vector units).
- * DEFMM_OPT_P2M_MFMA: the same for P2M (leaves of at most 64 points; larger
- * leaves stay on the vector units).  DEFMM_OPT_M2L_SLICED (orders <= 7): 1
+ * the mixed-precision path 16 or 8 right-hand sides at a time on the matrix
+ * cores when the plan's width allows it; 0 keeps it on the vector units (up to
+ * 8 right-hand sides per kernel value).  DEFMM_OPT_L2P_MFMA: 1 (default)
+ * evaluates L2P 16 right-hand sides per pass over a leaf's slots on the matrix
+ * cores; 0: one right-hand side per pass.  DEFMM_OPT_P2M_MFMA: the same for
+ * P2M (leaves of at most 64 points; larger leaves take one right-hand side per
+ * pass).  DEFMM_OPT_M2L_SLICED (orders <= 7): 1
  * sweeps each M2L work group's sources once per slice of its frequencies
  * (a work group then reads a third of each row at a time, so rows shared
  * with neighbouring work groups stay in L2 longer); 0 (default) sweeps them
