@@ -791,11 +791,14 @@ struct M2LShape {
 // loads 31).  It holds G x NW x V x NR accumulators, at most 16 (double) or 32
 // (float) complex; of the NW that allow that, the largest with blocks of at
 // least two waves, none of them mostly idle.
+// Order 2 loads one value a lane: in float its 27 would leave 14 lanes of the
+// wave (200,000-point sphere, 8 right-hand sides, 4.75 ms, so 3.22; 30,000
+// clustered points, one, 0.066 and 0.058).
 template <typename R, int L, int NR>
 struct M2LShapeN {
   static constexpr int PP = M2LShape<L>::PP;
   static constexpr int G = M2LShape<L>::G;
-  static constexpr int V = 16 / (2 * (int)sizeof(R));
+  static constexpr int V = L == 2 ? 1 : 16 / (2 * (int)sizeof(R));
   static constexpr int UN = (PP + V - 1) / V;  // units of a row
   static constexpr int tb(int nw) { return ((UN + nw - 1) / nw + 63) / 64 * 64; }
   static constexpr bool fits(int nw) {
@@ -807,8 +810,11 @@ struct M2LShapeN {
 };
 // Right-hand sides per M2L launch: at most 16 (double) or 32 (float)
 // complex accumulators per thread.
-// (double from L = 7: one, float at L = 7: two; wider kernels spill at the
-// occupancy asked for below, and at L = 8 in double without it)
+// (double: 4 up to order 3, 2 at 4, then one.  Float: 8 at order 2, then 4,
+// two from order 5 on; at order 3 8 would take the 200,000-point sphere from
+// 7.5 to 7.0 ms, but the 20,000-point cube from 0.182 to 0.187, 100,000
+// clustered points from 0.33 to 0.36 and the 8,000-point cube from 0.061 to
+// 0.079.)
 template <typename R, int L>
 constexpr int m2lMaxNR() {
   if (M2LShape<L>::kColumns) return sizeof(R) == 8 ? 1 : 2;
@@ -816,7 +822,7 @@ constexpr int m2lMaxNR() {
     constexpr int cap = 16 / (M2LShape<L>::G * M2LShape<L>::NW);
     return L >= 7 ? 1 : cap >= 4 ? 4 : cap >= 2 ? 2 : 1;
   }
-  return L <= 4 ? 4 : 2;
+  return L == 2 ? 8 : L <= 4 ? 4 : 2;
 }
 static int m2lMaxNRAt(int prec, int L) {
   switch (L) {
@@ -911,7 +917,7 @@ __global__ __launch_bounds__((M2LShapeN<R, L, NR>::TB)) void k_m2l(
   constexpr int P = 2 * L - 1, LL = L * L * L, PP = P * P * P;
   typedef M2LShapeN<R, L, NR> Sh;
   constexpr int NW = Sh::NW, TB = Sh::TB, G = Sh::G, V = Sh::V, RS = rowStride<R, L>();
-  struct alignas(16) Vec {
+  struct alignas(sizeof(R2) * V) Vec {
     R2 v[V];
   };
   constexpr int NU = G * NR, NB = f2lBatch(NU);
