@@ -4,9 +4,9 @@
 //   M_s[I] = conj(sig2_s[I]) sum_j S_I(y_j) W_s[j],  W_s[j] = q_j exp(-i kappa d_s.(y_j - c))
 //   p_i   += sum_s exp(i kappa d_s.(x_i - c)) sum_I S_I(x_i) (sig2_s[I] L_s[I])
 // The Lagrange weights S are real and the same for all of a leaf's slots, so
-// both are products of a real matrix with 16 slots' complex columns:
-// V_MFMA_F64_16X16X4_F64 or V_MFMA_F32_16X16X4_F32, one each for the real and
-// the imaginary part.  Operand layouts (A 16 x 4, B 4 x 16, D 16 x 16): lane
+// both are products of a real matrix with 16 slots' complex columns (L2P) or
+// rows (P2M): V_MFMA_F64_16X16X4_F64 or V_MFMA_F32_16X16X4_F32, one each for
+// the real and the imaginary part.  Operand layouts (A 16 x 4, B 4 x 16, D 16 x 16): lane
 // l holds A[l % 16][l / 16] and B[l / 16][l % 16]; D column l % 16, and row
 // 4 (l / 16) + v (float) or 4 v + l / 16 (double) in register v.
 #pragma once
@@ -60,16 +60,22 @@ __device__ __forceinline__ void stageWeights(R (&Wt)[3][NP][L], double (&rel)[3]
   }
 }
 
-// P2M.  A wave per (leaf, 16 slots).  The leaf's points are taken 64 at a time: a lane forms the charges
-// W of its slot at 16 of them (B operands, kept in registers) and every 16
-// rows of L^3 run ceil(n / 4) steps.  Points beyond the first 64 add to the
-// expansions that the wave itself has written.
+// P2M.  A wave per (leaf, 16 slots).  The leaf's points are taken 64 at a
+// time: a lane forms the charges W of its slot at 16 of them (A operands: slots
+// x points, kept in registers) and every 16 columns of L^3 run ceil(n / 4)
+// steps (B operands: the products of three weights).  Lane l ends with weight
+// index 16 m + l % 16 of four slots, so a store covers whole lines of 16
+// values.  Points beyond the first 64 add to the expansions that the wave
+// itself has written.
 //
 // Bound by writing the expansions (20,000 points, order 8, double: 0.8 GB,
 // 0.17 ms at the copy rate) and the latency of a wave's short chains.  Against
 // a thread per grid point over all points with weights and charges from LDS
-// (k_p2m): there 0.57 -> 0.33 ms, order 4 94 -> 52 us, 200,000-point sphere
-// order 5 3.7 -> 2.4 ms (double), 2.2 -> 1.7 ms (float).
+// (k_p2m): there 0.56 -> 0.29 ms, order 4 92 -> 52 us, 200,000-point sphere at
+// 64 wavelengths, order 5, 3.7 -> 2.5 ms (double), 2.2 -> 1.3 ms (float).  With
+// the operands the other way round (slots as columns: 8 bytes of every 32 a
+// store in float) 60,000 points, order 7, float, took 1.45 ms where this takes
+// 0.74 and k_p2m 1.19.
 template <typename R, int L>
 __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(3))) void k_p2m_slots(
     const int2* __restrict__ items, DevCells S, DevLevels lv, const double* __restrict__ px,
@@ -92,17 +98,19 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(3))) void k_
   const int hf = lv.isHF[lvl], doff = lv.dirOff[lvl], srow = lv.sigRow0[lvl];
   const int lane = threadIdx.x;
   const int lr = lane & 15, quad = lane >> 4;
-  const int kl = k0 + lr;  // this lane's column
-  const bool col = kl < ns;
-  const int sl = s0 + min(kl, ns - 1);
-  const int d = hf ? S.slotDir[sl] : 0;
+  // this lane's slot as an operand, and the directions of the four slots that
+  // it stores
+  const int d = hf ? S.slotDir[s0 + min(k0 + lr, ns - 1)] : 0;
+  int dirOf[4];
+#pragma unroll
+  for (int v = 0; v < 4; v++)
+    dirOf[v] = hf ? S.slotDir[s0 + min(k0 + X::row(quad, v), ns - 1)] : 0;
   double dx = 0., dy = 0., dz = 0.;
   if (hf) {
     dx = dirs[3 * (doff + d)];
     dy = dirs[3 * (doff + d) + 1];
     dz = dirs[3 * (doff + d) + 2];
   }
-  const R2* sgr = hf ? sig2 + (size_t)(srow + d) * LL : sig2;
   for (int j0 = 0; j0 < n; j0 += NP) {
     const int cn = min(NP, n - j0);
     if (j0 > 0) __syncthreads();
@@ -129,29 +137,45 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(3))) void k_
     // registers beside the slot's charges)
 #pragma unroll 1
     for (int mt = 0; mt < MT; mt++) {
-      const int I = min(16 * mt + lr, LL - 1);  // (rows beyond LL are not stored)
+      const int I = min(16 * mt + lr, LL - 1);  // (columns beyond LL are not stored)
       const int a0 = I / (L * L), a1 = (I / L) % L, a2 = I % L;
+      // (in float the epilogue's operands are loaded ahead of the steps; in
+      // double they would not fit the registers)
+      constexpr bool kAhead = sizeof(R) == 4;
+      auto phase = [&](int v) { return sig2[(size_t)(srow + dirOf[v]) * LL + I]; };
+      auto out = [&](int v) { return M + (size_t)(s0 + k0) * LL + X::row(quad, v) * LL + I; };
+      R2 sg[kAhead ? 4 : 1], old[kAhead ? 4 : 1];
+      if constexpr (kAhead)
+#pragma unroll
+        for (int v = 0; v < 4; v++) {
+          if (hf) sg[v] = phase(v);
+          if (j0 > 0 && k0 + X::row(quad, v) < ns) old[v] = *out(v);
+        }
       typename X::V dre = {0, 0, 0, 0}, dim = {0, 0, 0, 0};
 #pragma unroll
       for (int ks = 0; ks < KS; ks++) {
         if (ks >= ksn) break;
         const int j = 4 * ks + quad;
         const R a = Wt[0][j][a0] * Wt[1][j][a1] * Wt[2][j][a2];
-        dre = X::mac(a, br[ks], dre);
-        dim = X::mac(a, bi[ks], dim);
+        dre = X::mac(br[ks], a, dre);
+        dim = X::mac(bi[ks], a, dim);
       }
-      if (col) {
+      if (16 * mt + lr < LL) {
 #pragma unroll
         for (int v = 0; v < 4; v++) {
-          const int Io = 16 * mt + X::row(quad, v);
-          if (Io < LL) {
+          if (k0 + X::row(quad, v) < ns) {
             R2 val = c2<R>(dre[v], dim[v]);
-            if (hf) val = cmulc(val, sgr[Io]);
-            R2* o = M + (size_t)sl * LL + Io;
+            R2* o = out(v);
+            if (hf) {
+              if constexpr (kAhead) val = cmulc(val, sg[v]);
+              else val = cmulc(val, phase(v));
+            }
             if (j0 > 0) {
-              const R2 old = *o;
-              val.x += old.x;
-              val.y += old.y;
+              R2 was;
+              if constexpr (kAhead) was = old[v];
+              else was = *o;
+              val.x += was.x;
+              val.y += was.y;
             }
             *o = val;
           }
