@@ -1829,6 +1829,7 @@ struct Exec {
     gSrc = bRows = nullptr;
     partial = qio = pio = nullptr;
     phaseTab = nullptr;
+    l2p = nullptr;
     l2pItems = nullptr;
     l2pShared = nullptr;
     l2pPartial = nullptr;
@@ -2106,17 +2107,32 @@ static int uploadTyped(Exec& X) {
     X.phaseTab = d;
   }
   {
-    // L2P items: tiles of at most TP points, the slots in equal ranges of at
+    // L2P: leaves of few slots go to the vector kernel (k_l2p), the others in
+    // items of a tile of at most TP points and the slots in equal ranges of at
     // most `per` (multiples of 16); half as many where that leaves the chip
     // idle
     const int TP = l2pSlotTileAt(L, (int)sizeof(R));
+    const bool small = X.hL2PLeaf.size() < 2048;
+    const int slotsMin = l2pSlotsMin(L, (int)sizeof(R), small);
+    int64_t slots = 0;
+    for (const auto& lf : X.hL2PLeaf) slots += lf.ns;
+    const bool enough = slots >= slotsMin * (int64_t)X.hL2PLeaf.size();
+    std::vector<int> few;
+    std::vector<Exec::LeafSlots> cols;
+    for (const auto& lf : X.hL2PLeaf) {
+      if (lf.ns == 0) continue;
+      if (small ? enough : lf.ns >= slotsMin) cols.push_back(lf);
+      else few.push_back(lf.cell);
+    }
+    CKR(X.upv(X.l2p, few));
+    X.nl2p = (int)few.size();
     std::vector<L2PItem> items;
     std::vector<L2PTile> shared;
     for (int per = kL2PSlots;; per /= 2) {
       items.clear();
       shared.clear();
       int out = 0;
-      for (const auto& lf : X.hL2PLeaf) {
+      for (const auto& lf : cols) {
         const int tiles = (lf.n + TP - 1) / TP, nt = (lf.n + tiles - 1) / tiles;
         const int parts = (lf.ns + per - 1) / per;
         const int len = ((lf.ns + parts - 1) / parts + kSlotCols - 1) / kSlotCols * kSlotCols;
@@ -2320,18 +2336,8 @@ static int upload(Exec& X, Plan& pl) {
     CKR(X.upv(X.p2mBigSlotItems, it.bigSlots));
     X.np2mBigSlot = (int)it.bigSlots.size();
   }
-  {
-    // L2P leaves of few slots (k_l2p); the others are cut into items at the
-    // typed upload (their tiles depend on the precision)
-    std::vector<int> few;
-    for (int c : pl.l2pCell) {
-      const int ns = pl.T.nslot[c];
-      if (ns >= l2pSlotsMin(pl.l2pCell.size())) X.hL2PLeaf.push_back({c, pl.T.nprt[c], ns, pl.T.pbeg[c]});
-      else few.push_back(c);
-    }
-    CKR(X.upv(X.l2p, few));
-    X.nl2p = (int)few.size();
-  }
+  for (int c : pl.l2pCell)
+    X.hL2PLeaf.push_back({c, pl.T.nprt[c], pl.T.nslot[c], pl.T.pbeg[c]});
   {
     // tiles of the matrix-core L2P: 32 points up to L^3 = 512, else 16
     const int tp = pl.LL <= 512 ? 32 : 16;
