@@ -2505,8 +2505,20 @@ static void launchM2L(Exec& X, hipStream_t s, int g0, int ng, int chunks,
   constexpr int G = M2LShapeN<R, L, NR>::G;
   int64_t grid = 0;
   const XcdParts parts = m2lParts(X, g0, ng, chunks, grid);
+  // LDS that keeps a CU to one block where groups are long: their blocks, in
+  // step over the same offsets, read more rows at a time than the L2 holds.
+  // Float, orders 9 and 10, one right-hand side (384 threads at 126 registers
+  // fit twice): 100,000 clustered points, kappa = 0, order 10, 85 entries a
+  // group, 7.66 -> 5.55 ms; 36 entries 0.67 -> 0.55; but 17 entries 2.33 ->
+  // 2.53 and 7 entries 2.44 -> 2.94.
+  unsigned lds = 0;
+  if constexpr (sizeof(R) == 4 && NR == 1 && L >= 9) {
+    constexpr unsigned P = 2 * L - 1, used = (L * P * P + L * L * P) * sizeof(R2);
+    static_assert(used < 98304, "one block a CU");
+    if (X.hGroupBeg[g0 + ng] - X.hGroupBeg[g0] >= 32 * (int64_t)ng) lds = 98304 - used;
+  }
   auto go = [&](auto kernel, int tb) {
-    hipLaunchKernelGGL(kernel, itemGrid(grid), dim3(tb), 0, s, X.gBeg + g0,
+    hipLaunchKernelGGL(kernel, itemGrid(grid), dim3(tb), lds, s, X.gBeg + g0,
                        X.gTarget + (size_t)g0 * G, X.gSrc, X.gMask, X.gCode, F, X.fStride,
                        (const R2*)X.U, Lb, X.lStride, oc.twc, oc.tws, parts);
   };

@@ -1,6 +1,8 @@
-"""M2L at order 2 (one value a lane, up to 8 right-hand sides a launch): far
-fields are compared with the oracle's, batches with single evaluations, at the
-bounds of the other comparisons of that kind."""
+"""M2L block shapes that depend on the order and on the groups' length: order 2
+(one value a lane, up to 8 right-hand sides a launch) and long groups at orders
+9 and 10 (one block a CU for one right-hand side in float).  Far fields are
+compared with the oracle's, batches with single evaluations, at the bounds of
+the other comparisons of that kind."""
 import sys
 
 import numpy as np
@@ -67,3 +69,26 @@ def test_order_2_batches_match_single(nr):
             print(f"  precision {prec}: rel L2 {l2:.3e} max {mx:.3e}", flush=True)
             assert l2 <= tol and mx <= 10 * tol
     sys.stdout.flush()
+
+
+@pytest.mark.parametrize("L", [9, 10])
+@pytest.mark.parametrize("n,ncrit,nl,long", [(15000, 65, 0, True), (4000, 40, 5, False)])
+def test_long_groups_match_pairs(L, n, ncrit, nl, long):
+    """A pair takes another shape than its members, with the same sums."""
+    import defmm_amd as dm
+    from defmm_amd import workloads as wl
+    pts = wl.GEOMETRIES["clusters"](n, seed=3)
+    kappa = wl.kappa_for(nl, pts) if nl else 0.0
+    Q = np.stack([wl.charges(n, seed=70 + r) for r in range(2)])
+    print(f"case: clusters N={n} {nl} wavelengths L={L}, one right-hand side and two", flush=True)
+    A = _plan(dm, pts, L, ncrit, kappa, dm.MIXED)
+    s = A.stats()
+    assert (s["m2l_group_entries"] >= 32 * s["m2l_groups"]) == long
+    single = np.stack([A.apply(q) for q in Q])
+    A.set_rhs(2)
+    P = A.apply_batch(Q)
+    A.destroy()
+    l2, mx = _diff(P, single)
+    print(f"  rel L2 {l2:.3e} max {mx:.3e}", flush=True)
+    sys.stdout.flush()
+    assert l2 <= 1e-6 and mx <= 1e-5
