@@ -71,18 +71,30 @@ def log(msg):
 
 
 def m2l_nr_per_launch(L, mixed):
-    """Right-hand sides that share one read of a table row in M2L (the
-    executor's rule: at most 16 double or 32 float complex accumulators per
-    thread, less where that spills; a launch of the stored variant covers up
-    to 8 such chunks one after another)."""
+    """Right-hand sides that share one read of a table row in M2L, at most
+    (the executor's rule: at most 16 double or 32 float complex accumulators
+    per thread, less where that spills)."""
     if mixed:
-        return 4 if L <= 4 else 2
+        return 8 if L == 2 else 4 if L <= 4 else 2
     if L >= 7:
         return 1
     PP = (2 * L - 1) ** 3
     nw = max(-(-PP // 1024), min(-(-PP // 256), 3))
     cap = 16 // (4 * nw)
     return 4 if cap >= 4 else 2 if cap >= 2 else 1
+
+
+def m2l_launches(L, nrhs, mixed, batched=False):
+    """M2L launches over all groups: each takes the widest chunk of 8, 4, 2 or 1
+    right-hand sides that the order allows, in the stored variant up to 8 such
+    chunks (the batched variant's workspace holds one, and each of its launches
+    is cut into the plan's batches)."""
+    left, launches = nrhs, 0
+    while left:
+        w = next(w for w in (8, 4, 2, 1) if w <= min(left, m2l_nr_per_launch(L, mixed)))
+        left -= w * (1 if batched else min(8, left // w))
+        launches += 1
+    return launches
 
 
 def m2l_compulsory_bytes(st, L, nrhs, mixed, batched=False):
@@ -95,8 +107,7 @@ def m2l_compulsory_bytes(st, L, nrhs, mixed, batched=False):
     PP, LL = (2 * L - 1) ** 3, L ** 3
     s = 8 if mixed else 16
     g = 1 if L >= 8 else 3 if L == 7 else 4
-    nr = m2l_nr_per_launch(L, mixed)
-    launches = -(-nrhs // nr)
+    launches = m2l_launches(L, nrhs, mixed, batched)
     lists = st["m2l_group_entries"] * (4 + 4 + 4 * g) + st["m2l_groups"] * (4 + 4 * g)
     per_rhs = st["m2f_slots"] * (LL if batched else PP) * s + st["m2l_targets"] * LL * s
     per_launch = st["m2l_table_rows"] * PP * s + lists
