@@ -2406,7 +2406,6 @@ static int upload(Exec& X, Plan& pl) {
     CKR(buildP2PItems(pl, kP2PMfmaTargets, items, beg, g_err));
     X.nitems = (int)items.size();
     X.nleaves = (int)pl.p2pLeaf.size();
-    X.st.p2p_items = X.nitems;
     CKR(X.upv(X.items, items));
     CKR(X.upv(X.itemBeg, beg));
   }
@@ -3021,11 +3020,15 @@ int defmm_plan_set_rhs(defmm_plan plan, int nrhs) {
 int defmm_plan_stats(defmm_plan plan, int64_t* out, int n) {
   if (!plan || !out) { g_err = "null argument"; return DEFMM_EARG; }
   const dfm::Stats& s = plan->x.st;
+  // near-field items of the kernel that the plan's precision and width take
+  const Exec& X = plan->x;
+  const int64_t p2pItems =
+      X.prec == DEFMM_MIXED && X.nr >= 8 && X.p2pMfma ? X.nitems : X.nLaneItems;
   int64_t v[DEFMM_NSTATS] = {s.p2p_calls, s.p2p_pairs, s.hf_m2l, s.lf_m2l, s.src_slots,
                              s.trg_slots, s.hf_tables, s.lf_tables, s.hf_leaves_p2m,
                              s.lf_leaves_p2m, s.hf_m2m, s.lf2hf_m2m, s.lf_m2m, s.hf_l2p,
                              s.lf_l2p, s.hf_l2l, s.hf2lf_l2l, s.lf_l2l, s.nlvl, s.cpt,
-                             s.max_stage, s.ncells_t, s.ncells_s, s.p2p_items, s.m2f_slots,
+                             s.max_stage, s.ncells_t, s.ncells_s, p2pItems, s.m2f_slots,
                              s.m2l_entries, s.m2l_targets, s.m2l_groups,
                              s.m2l_group_entries, s.m2l_batches, s.m2l_batch_rows,
                              s.ms_tree, s.ms_walk, s.ms_tables, s.ms_trans, s.ms_m2l,

@@ -95,7 +95,7 @@ struct Stats {
   int64_t hf_m2m = 0, lf2hf_m2m = 0, lf_m2m = 0, hf_l2p = 0, lf_l2p = 0;
   int64_t hf_l2l = 0, hf2lf_l2l = 0, lf_l2l = 0, nlvl = 0, cpt = 0, max_stage = 0;
   int64_t ncells_t = 0, ncells_s = 0;
-  int64_t p2p_items = 0, m2f_slots = 0, m2l_entries = 0, m2l_targets = 0;
+  int64_t m2f_slots = 0, m2l_entries = 0, m2l_targets = 0;
   int64_t m2l_groups = 0, m2l_group_entries = 0;
   int64_t m2l_batches = 0, m2l_batch_rows = 0;  // batched M2L (set at upload)
   // host set-up time per phase (ms): trees, dual walk, kernel tables and
