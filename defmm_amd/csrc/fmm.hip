@@ -2329,8 +2329,8 @@ static int upload(Exec& X, Plan& pl) {
     // (table id << 6 | h) -> row of the materialised table store << 3: one
     // row per (table, axis order, flips) that some entry reads, in key order
     // (codes of absent group targets point at row 0, never read).  Marking
-    // the keys in use and mapping the codes run in parallel over ranges of
-    // entries; the result does not depend on the thread count.
+    // the keys in use, mapping the codes and the groups' costs run in parallel
+    // over ranges; the result does not depend on the thread count.
     const size_t nkeys = (size_t)std::max(1, pl.ntab) * 48;
     const int G = pl.m2lG;
     const size_t ne = pl.m2lGMask.size();
@@ -2338,15 +2338,15 @@ static int upload(Exec& X, Plan& pl) {
       return ((size_t)(c >> 6) * 6 + kVariantOfSigma[(c >> 3) & 7]) * 8 + (c & 7);
     };
     const unsigned nth = std::max(1u, std::min(32u, std::thread::hardware_concurrency()));
-    auto parallel = [&](auto&& fn) {
+    auto parallel = [&](size_t n, auto&& fn) {
       std::vector<std::thread> th;
-      for (unsigned t = 0; t < nth; t++) th.emplace_back(fn, ne * t / nth, ne * (t + 1) / nth, t);
+      for (unsigned t = 0; t < nth; t++) th.emplace_back(fn, n * t / nth, n * (t + 1) / nth, t);
       for (auto& x : th) x.join();
     };
     // per-thread marks of the keys in use (no shared writes), then merged
     std::vector<std::vector<uint8_t>> used(nth);
     std::vector<int> bad(nth, 0);
-    parallel([&](size_t e0, size_t e1, unsigned t) {
+    parallel(ne, [&](size_t e0, size_t e1, unsigned t) {
       used[t].assign(nkeys, 0);
       for (size_t e = e0; e < e1; e++)
         for (int g = 0; g < G; g++)
@@ -2373,23 +2373,26 @@ static int upload(Exec& X, Plan& pl) {
     }
     std::vector<std::vector<uint8_t>>().swap(used);
     ListVec dc(pl.m2lGCode.size());  // every element written below
-    parallel([&](size_t e0, size_t e1, unsigned) {
-      for (size_t e = e0; e < e1; e++)
-        for (int g = 0; g < G; g++)
-          dc[e * G + g] = ((pl.m2lGMask[e] >> g) & 1) ? rowOf[keyOf(pl.m2lGCode[e * G + g])] << 3 : 0;
+    // beside the codes, the groups' rows to load (summed up below)
+    X.hGroupCost.assign(pl.m2lGroupBeg.size(), 0);
+    parallel((size_t)X.nGroups, [&](size_t g0, size_t g1, unsigned) {
+      for (size_t grp = g0; grp < g1; grp++) {
+        int64_t rows = 4;
+        for (size_t e = pl.m2lGroupBeg[grp]; e < (size_t)pl.m2lGroupBeg[grp + 1]; e++) {
+          rows++;
+          for (int g = 0; g < G; g++) {
+            const bool on = (pl.m2lGMask[e] >> g) & 1;
+            rows += on;
+            dc[e * G + g] = on ? rowOf[keyOf(pl.m2lGCode[e * G + g])] << 3 : 0;
+          }
+        }
+        X.hGroupCost[grp + 1] = rows;
+      }
     });
+    for (int g = 0; g < X.nGroups; g++) X.hGroupCost[g + 1] += X.hGroupCost[g];
     if (X.hRowKey.empty()) X.hRowKey.push_back(0);
     X.st.m2l_table_rows = (int64_t)X.hRowKey.size();
     CKR(X.upv(X.gCode, dc));
-  }
-  {
-    X.hGroupCost.assign(pl.m2lGroupBeg.size(), 0);
-    for (int g = 0; g < X.nGroups; g++) {
-      int64_t c = 4;
-      for (int e = pl.m2lGroupBeg[g]; e < pl.m2lGroupBeg[g + 1]; e++)
-        c += 1 + __builtin_popcount((unsigned)pl.m2lGMask[e]);
-      X.hGroupCost[g + 1] = X.hGroupCost[g] + c;
-    }
   }
   X.hGSrcF.swap(pl.m2lGSrcF);
   X.hM2fSlot = pl.m2fSlot;
@@ -2397,13 +2400,14 @@ static int upload(Exec& X, Plan& pl) {
   {
     std::vector<P2PItem> items;
     std::vector<int> beg;
-    CKR(buildP2PItems(pl, kP2PTargets, items, beg, g_err));
+    const NearLists lists = nearLists(pl);
+    CKR(buildP2PItems(pl, lists, kP2PTargets, items, beg, g_err));
     X.nLaneItems = (int)items.size();
     CKR(X.upv(X.laneItems, items));
     CKR(X.upv(X.laneItemBeg, beg));
     items.clear();
     beg.clear();
-    CKR(buildP2PItems(pl, kP2PMfmaTargets, items, beg, g_err));
+    CKR(buildP2PItems(pl, lists, kP2PMfmaTargets, items, beg, g_err));
     X.nitems = (int)items.size();
     X.nleaves = (int)pl.p2pLeaf.size();
     CKR(X.upv(X.items, items));

@@ -44,10 +44,11 @@ int main() {
       failed++;
       continue;
     }
+    const NearLists lists = nearLists(pl);
     for (int tg : {kP2PTargets, kP2PMfmaTargets}) {
       std::vector<P2PItem> items;
       std::vector<int> beg;
-      rc = buildP2PItems(pl, tg, items, beg, msg);
+      rc = buildP2PItems(pl, lists, tg, items, beg, msg);
       int wrong = rc != OK;
       for (size_t lf = 0; lf < pl.p2pLeaf.size() && !wrong; lf++) {
         const int n = pl.T.nprt[pl.p2pLeaf[lf]];
@@ -87,9 +88,9 @@ int main() {
             break;
         }
         tried++;
-        missed += checkP2PItems(pl, tg, bad, badBeg).empty();
+        missed += checkP2PItems(pl, lists, tg, bad, badBeg).empty();
       }
-      const bool ok = !wrong && !missed && checkP2PItems(pl, tg, items, beg).empty();
+      const bool ok = !wrong && !missed && checkP2PItems(pl, lists, tg, items, beg).empty();
       std::printf("case %s %d %s leaves %zu items %zu wrong %d tried %d missed %d\n", c.name, tg,
                   ok ? "OK" : "FAIL", pl.p2pLeaf.size(), items.size(), wrong, tried, missed);
       failed += !ok;

@@ -22,9 +22,9 @@ pytestmark = pytest.mark.gpu
     ("sphere", 12000, 4000, 12, 6, 20),
     ("clusters", 9000, 0, 0, 6, 33),
     ("sphere", 8000, 0, 9, 7, 33),
-    ("cube_edges", 12000, 0, 14, 8, 40),
-    ("ellipsoid", 16000, 0, 24, 9, 33),
-    ("sphere", 7000, 0, 10, 10, 20),
+    ("cube_edges", 8000, 0, 10, 8, 33),
+    ("ellipsoid", 7000, 0, 24, 9, 33),
+    ("sphere", 4000, 0, 8, 10, 18),
 ])
 def test_far_field_matches_oracle(geo, n, m, nl, L, ncrit):
     import defmm_amd as dm
