@@ -34,11 +34,13 @@ inline bool p2mOnColumns(int L, bool large, int64_t waves, int64_t blocks) {
 // (small: the mean over the plan's leaves counts), larger plans decide by
 // leaf.  Against the vector kernel, float and double, us: order 3, 5,000-point
 // cube (28 slots a leaf) 16 and 13, 29 and 15, 60,000-point sphere (178) 167
-// and 158, 410 and 250; order 5, 30,000-point ellipsoid (17) 36 and 46, 76 and
-// 58; order 8, 8,000-point ellipsoid (4) 57 and 37, 72 and 56, 5,000-point cube
-// 74 and 88, 84 and 140, 20,000-point cube (81) 226 and 420, 308 and 690.  The
-// vector kernel's staging does not fit its LDS well at order 9 in float and 10
-// in double (8,000-point ellipsoid 57 and 94, 196 and 312).
+// and 158, 410 and 250; order 4, 5,000-point cube 16 and 18, 29 and 21,
+// 4,000-point cube (36) 16 and 21, 18 and 25; order 5, 30,000-point ellipsoid
+// (17) 36 and 46, 76 and 58; order 8, 8,000-point ellipsoid (4) 57 and 37, 72
+// and 56, 5,000-point cube 74 and 88, 84 and 140, 20,000-point cube (81) 226
+// and 420, 308 and 690.  The vector kernel's staging does not fit its LDS well
+// at order 9 in float and 10 in double (8,000-point ellipsoid 57 and 94, 196
+// and 312).
 inline int l2pSlotsMin(int L, int realBytes, bool small) {
   const bool f = realBytes == 4;
   constexpr int never = INT32_MAX;
@@ -46,7 +48,7 @@ inline int l2pSlotsMin(int L, int realBytes, bool small) {
   if (L == 3) return f && small ? 48 : never;
   if (L == (f ? 9 : 10)) return 3;
   if (!small) return 24;
-  if (L == 4) return 48;
+  if (L == 4) return f ? 24 : 32;
   return f || L >= 7 ? 12 : L == 6 ? 24 : 32;
 }
 
