@@ -4,8 +4,8 @@
 #pragma once
 #include <algorithm>
 #include <cstdint>
+#include <exception>
 #include <string>
-#include <system_error>
 #include <thread>
 #include <vector>
 
@@ -55,11 +55,12 @@ inline NearLists nearLists(const Plan& pl) {
   const size_t nth = std::max<size_t>(
       1, std::min<size_t>({16, std::thread::hardware_concurrency(), pl.p2pSrcB.size() / 65536}));
   std::vector<std::thread> th;
+  th.reserve(nth);
   size_t begun = 1;
   try {
     for (; begun < nth; begun++)
       th.emplace_back(fill, nl * begun / nth, nl * (begun + 1) / nth);
-  } catch (const std::system_error&) {  // no more threads: the rest here
+  } catch (const std::exception&) {  // no more threads or memory: the rest here
     fill(nl * begun / nth, nl);
   }
   fill(0, nl / nth);
