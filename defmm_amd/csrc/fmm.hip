@@ -1722,7 +1722,7 @@ struct Exec {
   int* laneItemBeg = nullptr;
   int p2pPhase = kPhaseLibrary;
   PhaseConsts phaseConsts{};
-  void* phaseTab = nullptr;  // kPhaseN complex values, plan's real type
+  void* phaseTab = nullptr;  // kPhaseN entries (PhaseT), plan's real type
   int *leafCell = nullptr, *itemBeg = nullptr, *rb = nullptr, *re = nullptr;
   int nleaves = 0;
   double2* partial = nullptr;
@@ -2049,13 +2049,12 @@ static int uploadTyped(Exec& X) {
     X.consts = d;
   }
   {
-    std::vector<R2> t(kPhaseN);
-    for (int k = 0; k < kPhaseN; k++) {
-      double c, sn;
-      phaseEntry(k, c, sn);
-      t[k] = c2h<R>(c, sn);
-    }
-    R2* d;
+    typedef typename PhaseT<R>::T E;
+    std::vector<E> t(kPhaseN);
+    if constexpr (sizeof(R) == 8)
+      for (int k = 0; k < kPhaseN; k++) phaseEntry(k, t[k].x, t[k].y);
+    else phaseEntriesF(t.data());
+    E* d;
     CKR(X.upv(d, t));
     X.phaseTab = d;
   }
@@ -2503,7 +2502,7 @@ static void launchP2PLane(Exec& X, hipStream_t s, int r0) {
     hipLaunchKernelGGL((k_p2p_lane<R, NR, decltype(phase)::value>),
                        itemGrid(((int64_t)X.nLaneItems + 3) / 4), dim3(256), 0, s, X.laneItems,
                        X.leafCell, X.T.pbeg, X.tx, X.ty, X.tz, X.sx, X.sy, X.sz, q, (size_t)X.ns,
-                       X.rb, X.re, (const R2*)X.phaseTab, X.phaseConsts, X.partial,
+                       X.rb, X.re, (const typename PhaseT<R>::T*)X.phaseTab, X.phaseConsts, X.partial,
                        X.nLaneItems);
   };
   if (X.p2pPhase == kPhaseNone) go(std::integral_constant<int, kPhaseNone>());
@@ -2520,7 +2519,7 @@ static void launchP2PMfma(Exec& X, hipStream_t s, int r0) {
   const float2* q = (const float2*)X.q + (size_t)r0 * X.ns;
   float2* p = (float2*)X.p + (size_t)r0 * X.nt;
   const P2PMfmaArgs A = {X.items, X.leafCell, X.T.pbeg, X.tx,  X.ty, X.tz, X.sx, X.sy, X.sz, q,
-                         (size_t)X.ns, X.rb, X.re, (const float2*)X.phaseTab, X.partial,
+                         (size_t)X.ns, X.rb, X.re, (const float4*)X.phaseTab, X.partial,
                          X.nitems};
   auto go = [&](auto phase) {
     hipLaunchKernelGGL((k_p2p_mfma<decltype(phase)::value, NR>),

@@ -34,11 +34,21 @@ __device__ __forceinline__ void invDist(double R2, double& r, float& K) {
   r = fma(0.5, Kd * fma(-r0, r0, R2), r0);
 }
 
+// An entry of the phase table: cos and sin, in float with its angle's shift (z)
+template <typename R>
+struct PhaseT {
+  typedef float4 T;
+};
+template <>
+struct PhaseT<double> {
+  typedef double2 T;
+};
+
 // Kernel value without the factor 1 / (4 pi), which the caller applies to
 // its sums.
 template <int Phase, typename R>
 __device__ __forceinline__ void p2pValue(double x, double y, double z, const PhaseConsts& pc,
-                                         const typename C2T<R>::T* __restrict__ tab, R& co,
+                                         const typename PhaseT<R>::T* __restrict__ tab, R& co,
                                          R& si) {
   const double R2 = fma(z, z, fma(y, y, x * x));
   double r;
@@ -118,12 +128,12 @@ __global__ __launch_bounds__(256) void k_p2p_lane(
     const double* __restrict__ tz, const double* __restrict__ sx, const double* __restrict__ sy,
     const double* __restrict__ sz, const typename C2T<R>::T* __restrict__ q, size_t qStride,
     const int* __restrict__ rb, const int* __restrict__ re,
-    const typename C2T<R>::T* __restrict__ phase, PhaseConsts pc, double2* __restrict__ partial,
+    const typename PhaseT<R>::T* __restrict__ phase, PhaseConsts pc, double2* __restrict__ partial,
     int nItems) {
   typedef typename C2T<R>::T R2;
   constexpr int TC = p2pSweep<R, NR>();
   constexpr bool kFloat = sizeof(R) == 4;
-  __shared__ R2 tab[Phase == kPhaseTable ? kPhaseN : 1];
+  __shared__ typename PhaseT<R>::T tab[Phase == kPhaseTable ? kPhaseN : 1];
   if constexpr (Phase == kPhaseTable) {
     static_assert(kPhaseN == 256, "one table entry per thread");
     tab[threadIdx.x] = phase[threadIdx.x];
@@ -282,7 +292,7 @@ struct P2PMfmaArgs {
   const float2* q;
   size_t qStride;
   const int *rb, *re;
-  const float2* phase;
+  const float4* phase;
   double2* partial;
   int nItems;
 };
@@ -291,7 +301,7 @@ struct P2PMfmaArgs {
 // the operands (Q_re, -Q_im) and (Q_im, Q_re) of columns r and r + 8 (8).
 template <int Phase, int NR, int MB>
 __device__ __forceinline__ void p2pMfmaItem(const P2PMfmaArgs& A, const PhaseConsts& pc, int item,
-                                            const P2PItem& it, const float2* tab,
+                                            const P2PItem& it, const float4* tab,
                                             double (*lc)[16], float2 (*lq)[17]) {
   static_assert(NR == 16 || NR == 8, "columns of the result");
   typedef float v4f __attribute__((ext_vector_type(4)));
@@ -411,7 +421,7 @@ __device__ __forceinline__ void p2pMfmaItem(const P2PMfmaArgs& A, const PhaseCon
 // of instruction take)
 template <int Phase, int NR>
 __global__ __launch_bounds__(256, 4) void k_p2p_mfma(P2PMfmaArgs A, PhaseConsts pc) {
-  __shared__ float2 tab[Phase == kPhaseTable ? kPhaseN : 1];
+  __shared__ float4 tab[Phase == kPhaseTable ? kPhaseN : 1];
   __shared__ double lc[4][3][16];
   __shared__ float2 lq[4][16][17];
   if constexpr (Phase == kPhaseTable) {

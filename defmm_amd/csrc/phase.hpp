@@ -65,6 +65,41 @@ inline void phaseEntry(int k, double& c, double& s) {
   s = (double)sinl(a);
 }
 
+// The float table's kPhaseN entries: x, y cos and sin of an angle
+// 2 pi k / kPhaseN + d, and z = -d, where d is the first of the searched ones
+// at which both lie within 2^-29 of a float (accurate tables, as in S. Gal,
+// "Computing elementary functions: a new approach for achieving high accuracy
+// and good performance", 1986).  An eighth of the circle is searched (0.1 ms),
+// the rest mirrored.
+constexpr double kPhaseShift = 3e-4;  // |d| at most
+template <typename T>
+inline void phaseEntriesF(T* tab) {
+  constexpr int Q = kPhaseN / 4;
+  constexpr double step = 3.1e-7, close = 1.0 / (1 << 29);
+  for (int k = 0; k <= Q / 2; k++) {
+    const double a = 6.283185307179586 / kPhaseN * k;
+    for (int j = 0; j * step / 2 < kPhaseShift; j++) {
+      const double d = (j & 1 ? -step : step) * ((j + 1) / 2), c = cos(a + d), s = sin(a + d);
+      tab[k].x = (float)c;
+      tab[k].y = (float)s;
+      tab[k].z = (float)-d;
+      if (std::fabs(tab[k].x - c) <= close && std::fabs(tab[k].y - s) <= close) break;
+    }
+  }
+  for (int k = Q / 2 + 1; k < Q; k++) {  // cos(pi / 2 - a) = sin(a)
+    const T e = tab[Q - k];
+    tab[k].x = e.y;
+    tab[k].y = e.x;
+    tab[k].z = -e.z;
+  }
+  for (int k = Q; k < kPhaseN; k++) {  // cos(a + pi / 2) = -sin(a)
+    const T e = tab[k - Q];
+    tab[k].x = -e.y;
+    tab[k].y = e.x;
+    tab[k].z = e.z;
+  }
+}
+
 // n mod kPhaseN of t = n + 1.5 * 2^52 (its low bits)
 DFM_HD inline int phaseIndex(double t) {
 #if defined(__HIP_DEVICE_COMPILE__)
@@ -96,23 +131,41 @@ DFM_HD inline void phaseTable(double r, double K, const PhaseConsts& pc, const T
   co = (e.x + fma(e.x, cm, -e.y * sy)) * K;
   si = (e.y + fma(e.y, cm, e.x * sy)) * K;
 }
-// Float values of a double r: the remainder is formed in double, then float
-// (|kappa y| <= pi / 256: the omitted y^5 / 120 and y^4 / 24 are below
-// 3e-12 and 1e-9).
-template <typename T2>
-DFM_HD inline void phaseTable(double r, float K, const PhaseConsts& pc, const T2* tab, float& co,
+// An entry's angle as its distance from 2 pi k / kPhaseN, negated; 0 where the
+// table holds cos and sin alone.
+template <typename T>
+DFM_HD inline auto phaseShift(const T& e, int) -> decltype(e.z) {
+  return e.z;
+}
+template <typename T>
+DFM_HD inline float phaseShift(const T&, long) {
+  return 0.f;
+}
+// Float values of a double r: the remainder is formed in double, then float,
+// the angle y from the entry's.  With 1 - cos y = sin y tan(y / 2), tan(y / 2)
+// as y / 2, the last sum alone rounds near 1 (|y| <= pi / 256 + 3e-4: the
+// omitted y^5 / 120 and y^4 / 24 are below 3e-12 and 1e-9): rms error 2.1e-8
+// at kappa = 201, where polynomials of the phase reduced by pi / 2 have 2.5e-8,
+// and 3.6e-8 was that of entries rounded at 2 pi k / kPhaseN with two sums near
+// 1, in as many instructions.  Of the float4 entries the kernels read all 16
+// bytes: 12 take LDS longer (200,000-point sphere at 40 wavelengths 5.67 and
+// 5.75 ms; a table of cos and sin and one of shifts 5.90; without shifts 5.52).
+template <typename T>
+DFM_HD inline void phaseTable(double r, float K, const PhaseConsts& pc, const T* tab, float& co,
                               float& si) {
   const double magic = 6755399441055744.0;
   const double t = fma(r, pc.inv, magic);
   const double n = t - magic;
   const int k = phaseIndex(t);
-  const float y = (float)fma(-n, pc.h, r) * pc.kf;
-  const float z = y * y;
-  const float sy = fmaf(z * -0.16666667f, y, y);
-  const float cm = -0.5f * z;
-  const T2 e = tab[k];
-  co = fmaf(-e.y, sy, fmaf(e.x, cm, e.x)) * K;
-  si = fmaf(e.x, sy, fmaf(e.y, cm, e.y)) * K;
+  const T e = tab[k];
+#if defined(__HIP_DEVICE_COMPILE__)
+  asm("" : : "v"(e.w));
+#endif
+  const float y = fmaf((float)fma(-n, pc.h, r), pc.kf, phaseShift(e, 0));
+  const float h = 0.5f * y;
+  const float sy = fmaf(y * y * -0.16666667f, y, y);
+  co = fmaf(-sy, fmaf(e.x, h, e.y), e.x) * K;
+  si = fmaf(sy, fmaf(-e.y, h, e.x), e.y) * K;
 }
 
 }  // namespace dfm
