@@ -268,8 +268,8 @@ __global__ __launch_bounds__(256) void k_p2p_lane(
 // share the source operands), 4 items per block with the phase table in LDS.
 // The wave stages 16 sources at a time in LDS of its own: lane l loads source
 // l % 16 (coordinate l / 16, and right-hand sides l / 16 + 4 u), one step
-// ahead; no barrier, so no wave waits for another.  Every 64 sources the sums
-// are added to double ones.
+// ahead; no barrier, so no wave waits for another.  Every 64 sources (8 of them
+// with 8 right-hand sides) the sums are added to double ones.
 //
 // Bound by the SIMD's issue: 64 pairs take the matrix core 128 clocks (16
 // right-hand sides; 64 for 8) and the vector unit about 200 (34 instructions,
@@ -283,7 +283,10 @@ __global__ __launch_bounds__(256) void k_p2p_lane(
 // lane per source 19.9 (two targets a sweep are too few for each source's
 // loads), with a lane per target and polynomials 16.3; 100,000 clustered
 // points without phase 0.17, 0.52 and 0.43; 5,000-point cube 0.073, 0.086 and
-// 0.111.
+// 0.111.  That was with sums of 64 sources (128 products in a chain) in float,
+// which left errors 1.1 to 2 times those of a lane per source (whole passes,
+// 20,000-point cube, order 8: 2.3e-7 and 1.45e-7); with 8 sources a sum it is
+// 1.34e-7, for 12.5 ms at the sphere.
 constexpr int kP2PMfmaNR = 16;
 struct P2PMfmaArgs {
   const P2PItem* items;
@@ -349,6 +352,17 @@ __device__ __forceinline__ void p2pMfmaItem(const P2PMfmaArgs& A, const PhaseCon
 #pragma unroll
     for (int u = 0; u < NR / 4; u++) nq[u] = ql[4 * u * A.qStride + j];
   };
+  auto flush = [&]() {
+#pragma unroll
+    for (int b = 0; b < MB; b++) {
+#pragma unroll
+      for (int v = 0; v < 4; v++) {
+        ar[b][v] += (double)dre[b][v];
+        if constexpr (NR == 16) ai[b][v] += (double)dim[b][v];
+      }
+      dre[b] = dim[b] = v4f{0.f, 0.f, 0.f, 0.f};
+    }
+  };
   advance(lr, lr);
   load();
   for (int pos = 0; pos < it.cnt; pos += kStage) {
@@ -392,18 +406,9 @@ __device__ __forceinline__ void p2pMfmaItem(const P2PMfmaArgs& A, const PhaseCon
             dim[b] = __builtin_amdgcn_mfma_f32_16x16x4f32(si, ch.x, dim[b], 0, 0, 0);
         }
       }
+      if (NR == 8 && k % 2 == 1) flush();
     }
-    if ((pos & 48) == 48 || pos + kStage >= it.cnt) {
-#pragma unroll
-      for (int b = 0; b < MB; b++) {
-#pragma unroll
-        for (int v = 0; v < 4; v++) {
-          ar[b][v] += (double)dre[b][v];
-          if constexpr (NR == 16) ai[b][v] += (double)dim[b][v];
-        }
-        dre[b] = dim[b] = v4f{0.f, 0.f, 0.f, 0.f};
-      }
-    }
+    if (NR == 16 && ((pos & 48) == 48 || pos + kStage >= it.cnt)) flush();
   }
   constexpr double kInv4Pi = 0.079577471545947667884;
 #pragma unroll
