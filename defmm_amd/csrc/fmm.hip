@@ -2065,7 +2065,7 @@ static int uploadTyped(Exec& X) {
     // idle
     const int TP = l2pSlotTileAt(L, (int)sizeof(R));
     const bool small = X.hL2PLeaf.size() < 2048;
-    const int slotsMin = l2pSlotsMin(L, (int)sizeof(R), small);
+    const int slotsMin = l2pSlotsMin(L, (int)sizeof(R), X.hL2PLeaf.size());
     int64_t slots = 0;
     for (const auto& lf : X.hL2PLeaf) slots += lf.ns;
     const bool enough = slots >= slotsMin * (int64_t)X.hL2PLeaf.size();
