@@ -318,7 +318,7 @@ class IBFMM_Mat:
     def set_option(self, option, value):
         """Execution option: OPT_P2P_MFMA, OPT_L2P_MFMA, OPT_P2M_MFMA (0 or 1:
         the stage of the mixed path on the matrix cores, 16 right-hand sides
-        at a time; 1 by default)."""
+        at a time, the near field also 8; 1 by default)."""
         self._need_plan()
         _check(lib().defmm_plan_set_option(self._plan, int(option), int(value)))
 

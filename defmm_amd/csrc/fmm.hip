@@ -2720,8 +2720,10 @@ static int runTyped(Exec& X, const double2* qin, double2* pout, int parts, int n
       } else if (sizeof(R) == 4 && n >= 8 && X.p2pMfma) {
         launchP2PMfma<8>(X, s, r0);
         r0 += 8;
-      } else if (sizeof(R) == 4 && n >= 8) { launchP2PLane<R, 8>(X, s, r0); r0 += 8; }
-      else if (n >= 4) { launchP2PLane<R, 4>(X, s, r0); r0 += 4; }
+      } else if (sizeof(R) == 4 && n >= 8) {
+        if constexpr (sizeof(R) == 4) launchP2PLane<R, 8>(X, s, r0);
+        r0 += 8;
+      } else if (n >= 4) { launchP2PLane<R, 4>(X, s, r0); r0 += 4; }
       else if (n == 3) { launchP2PLane<R, 3>(X, s, r0); r0 += 3; }
       else if (n >= 2) { launchP2PLane<R, 2>(X, s, r0); r0 += 2; }
       else { launchP2PLane<R, 1>(X, s, r0); r0 += 1; }

@@ -185,9 +185,10 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(3))) void k_
   }
 }
 
-// Points per tile of k_l2p_slots: the tile's S (points x L^3) in at most 64
-// KB of LDS (double: 32 points up to L = 6, 16 up to L = 10; float: 32 up to
-// L = 8).
+// Points per tile of k_l2p_slots: 32 where their S (points x L^3, without
+// padding) fits 64 KB (double up to order 6, float up to 8), else 16 whatever
+// they take: with padding 70, 95 and 132 KB in double at orders 8, 9 and 10, so
+// that one block fits a CU at the last two.
 template <typename R, int L>
 constexpr int l2pSlotTile() {
   return L * L * L * 32 * (int)sizeof(R) <= 65536 ? 32 : 16;
@@ -236,6 +237,7 @@ __global__ __launch_bounds__(256) void k_l2p_slots(
   constexpr int kB = l2pSlotChain(L);
   static_assert(kU % kB == 0, "chains end with a batch of loads");
   static_assert(ST >= 4 * KS, "rows of S hold the last step's padding");
+  static_assert(TP * ((ST + 3 * L) * sizeof(R) + 3 * 8 + 4 * 2 * sizeof(R)) <= 160 * 1024, "LDS");
   __shared__ R Sm[TP][ST];
   __shared__ R Wt[3][TP][L];
   __shared__ double rel[3][TP];
