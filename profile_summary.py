@@ -208,9 +208,12 @@ def cmd_counters(a):
     rs = rows(one(a.dir, "counter_collection.csv"))
     per = collections.defaultdict(lambda: collections.defaultdict(float))
     calls = collections.defaultdict(set)
+    ns = collections.defaultdict(float)
     for r in rs:
         k = short(r["Kernel_Name"])
         per[k][r["Counter_Name"]] += float(r["Counter_Value"])
+        if r["Dispatch_Id"] not in calls[k]:
+            ns[k] += float(r["End_Timestamp"]) - float(r["Start_Timestamp"])
         calls[k].add(r["Dispatch_Id"])
     names = sorted({c for v in per.values() for c in v})
     tanote = " (TA_BUSY_avr: averaged over TA instances, then summed)" if "TA_BUSY_avr" in names else ""
@@ -227,11 +230,12 @@ def cmd_counters(a):
     hit = "TCC_HIT_sum" in names and "TCC_MISS_sum" in names
     sq = "SQ_INSTS_VALU" in names
     if hit:
-        out += ["L2 hit = TCC_HIT_sum / (TCC_HIT_sum + TCC_MISS_sum); TA busy = TA_BUSY_avr / kernel cycles.", ""]
+        out += ["L2 hit = TCC_HIT_sum / (TCC_HIT_sum + TCC_MISS_sum); TA busy = TA_BUSY_avr / kernel cycles; "
+                "miss TB/s = 128 bytes x TCC_MISS_sum / the dispatches' time.", ""]
     head = f"{'kernel':44s} {'calls':>6s} " + " ".join(f"{c:>24s}" for c in names)
     ta = "TA_BUSY_avr" in names
     out.append(head + ("   MFMA busy  VALU busy" if sq else "") + ("  L2 hit" if hit else "")
-               + ("  TA busy" if ta else ""))
+               + ("  miss TB/s" if hit else "") + ("  TA busy" if ta else "") + "         ms")
     order = sorted(per, key=lambda k: -per[k].get("GRBM_GUI_ACTIVE", 0))
     for k in order[:a.top]:
         v = per[k]
@@ -244,10 +248,11 @@ def cmd_counters(a):
         if hit:
             hm = v.get("TCC_HIT_sum", 0) + v.get("TCC_MISS_sum", 0)
             row += f"  {100 * v.get('TCC_HIT_sum', 0) / hm:5.1f}%" if hm else "       -"
+            row += f"  {128 * v.get('TCC_MISS_sum', 0) / ns[k] / 1e3:9.2f}" if ns[k] else " " * 11
         if ta:
             cyc = v.get("GRBM_GUI_ACTIVE", 0) / a.xcds
             row += f"  {100 * v.get('TA_BUSY_avr', 0) / cyc:6.1f}%" if cyc else "        -"
-        out.append(row)
+        out.append(row + f"  {ns[k] / 1e6:9.3f}")
     open(a.out, "w").write("\n".join(out) + "\n")
     print(f"wrote {a.out}")
 
